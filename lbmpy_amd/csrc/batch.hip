@@ -64,6 +64,7 @@ __device__ __forceinline__ SweepArgs<TC> load_args(const CONST_AS SweepArgs<TC>*
   a.u_in = nullptr;
   a.nut_scale = TC(0);
   a.seed = 0;
+  a.order = XcdOrder::of(1);
   return a;
 }
 
@@ -121,7 +122,7 @@ batch_kernel(const BatchEntry<TC>* __restrict__ members, const int32_t* __restri
       const int x = (int)(local - row * nx);
       const uint32_t zz = row / ny;
       const int y = (int)(row - zz * ny);
-      sweep_cell<S, FAM, PAT, true, TS, TC>(a, x, y, (int)zz);
+      sweep_cell<S, FAM, PAT, true, true, TS, TC>(a, x, y, (int)zz);
     }
   }
 }

@@ -176,6 +176,37 @@ __device__ __forceinline__ float recip<float>(float x) {
   return __builtin_fmaf(r, __builtin_fmaf(-x, r, 1.0f), r);
 }
 
+// ---------------------------------------------------------------- cell numbering
+// Division of 0 <= n < 2^31 by a constant d >= 1 through a multiplication (Granlund and Montgomery 1994, N = 31):
+// with l = ceil(log2 d) and m = ceil(2^(31+l) / d) < 2^32, n / d = (n m) >> (31 + l).
+struct CellDivider {
+  uint32_t d, mul, shift;
+  __host__ __device__ static CellDivider of(uint32_t d) {
+    uint32_t l = 0;
+    while ((uint64_t(1) << l) < d) ++l;
+    return {d, (uint32_t)(((uint64_t(1) << (31 + l)) + d - 1) / d), 31 + l};
+  }
+  __host__ __device__ __forceinline__ uint32_t quotient(uint32_t n) const {
+    return (uint32_t)(((uint64_t)n * mul) >> shift);
+  }
+};
+
+// Consecutive workgroups go to the 8 XCDs in turn, each with an L2 of its own.  XcdOrder renumbers them so that runs of
+// `chunk` neighbouring block numbers share an XCD: within every group of 8 chunk blocks, the blocks of one XCD take
+// one run.  The blocks after the last whole group, and all of them with chunk <= 1, keep their numbers.
+struct XcdOrder {
+  uint32_t chunk;
+  CellDivider group;
+  __host__ __device__ static XcdOrder of(uint32_t chunk) {
+    if (chunk < 1) chunk = 1;
+    return {chunk, CellDivider::of(8 * chunk)};
+  }
+  __host__ __device__ __forceinline__ uint32_t number(uint32_t block, uint32_t blocks) const {
+    const uint32_t first = group.quotient(block) * group.d, k = block - first;
+    return first + group.d > blocks ? block : first + (k & 7) * chunk + (k >> 3);
+  }
+};
+
 // ---------------------------------------------------------------- launch arguments
 template <class TC>
 struct SweepArgs {
@@ -201,6 +232,8 @@ struct SweepArgs {
   const TC* u_in;             // moment family: equilibrium-velocity input
   TC nut_scale;               // 3/2 Cs^2
   uint32_t seed;              // stochastic FP16 rounding: this launch's seed
+  CellDivider row, plane;     // division by nx and by ny (thread_cell)
+  XcdOrder order;             // of the blocks (thread_cell)
 };
 
 // What a collision hands back to the cell beyond the populations: the Smagorinsky shear rate and Pi

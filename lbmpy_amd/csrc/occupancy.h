@@ -75,9 +75,13 @@ constexpr WaveCaps kWaveCaps[] = {
 // A launch's own waves_per_simd (1..8, or -1 for none) overrides the table: the best cap of the AA-odd kernels
 // differs from one MI355X to another (D3Q27 cumulant FP32 at 256^3: 0.607 ms at 2 waves and 0.664 at 3 on one,
 // 0.658 and 0.609 on another), and lbmpy_amd.sweep.tune_occupancy picks it by timing.
-inline int sweep_wave_cap(const lbm355_sweep_desc* d, bool staged, bool walls, unsigned block_threads) {
+// half_cache: the populations take less than half the Infinity Cache.  There the loads return sooner and the caps cost
+// 2-9% (D3Q27 cumulant FP32 64^3 10.0 -> 9.5 us without, D3Q19 TRT 96^3 with walls 25.2 -> 24.4, D3Q19 SRT 64^3 9.0 ->
+// 8.2); from there to 256 MiB they are even (128^3 56.1 and 56.2 us, with ghost layers 60.5 and 61.7).
+inline int sweep_wave_cap(const lbm355_sweep_desc* d, bool staged, bool walls, bool half_cache,
+                          unsigned block_threads) {
   if (d->waves_per_simd != 0) return d->waves_per_simd > 0 ? d->waves_per_simd : 0;
-  if (d->flags & LBM355_FLAG_LEARNED_CLOSURE) return 0;
+  if (half_cache || (d->flags & LBM355_FLAG_LEARNED_CLOSURE)) return 0;
   int kind;
   switch (d->pattern) {
     case LBM355_PULL: kind = CAP_PULL; break;

@@ -1,8 +1,8 @@
 // Fused stream-collide sweep for MI355X (gfx950) and its C ABI (include/lbm355.h).
 //
-// One thread per interior cell, x fastest (a 64-lane wavefront covers 64 consecutive cells of
-// one row, so each population is read and written as contiguous 256 B (FP32) segments).
-// Blocks span up to 256 cells of a row; the grid is (row blocks, ny, nz).  Streaming:
+// One thread per interior cell, x fastest (a 64-lane wavefront covers 64 consecutive cells, so each
+// population is read and written as contiguous 256 B (FP32) segments).  How the cells are numbered and
+// whether the accesses bypass the caches depends on size and alignment (sweep_launch).  Streaming:
 //   pull    read  src[i][x - c_i],        write dst[i][x]           (fieldaccess.py:66-75)
 //   AA even read  f[i][x],                write f[inv i][x]         (fieldaccess.py:136-145)
 //   AA odd  read  f[inv i][x - c_i],      write f[i][x + c_i]       (fieldaccess.py:148-157)
@@ -350,8 +350,8 @@ struct Launch {
   dim3 grid, block;
 };
 
-Launch geometry(int nx, int ny, int nz, bool rowlds = false) {
-  int bx = rowlds ? nx : (nx >= 256 ? 256 : ((nx + 63) / 64) * 64);
+Launch geometry(int nx, int ny, int nz) {
+  int bx = (nx >= 256 ? 256 : ((nx + 63) / 64) * 64);
   Launch l;
   l.block = dim3(bx, 1, 1);
   l.grid = dim3((nx + bx - 1) / bx, ny, nz);
@@ -362,7 +362,7 @@ size_t elem_size(int dtype) { return dtype == LBM355_F64 ? 8 : (dtype == LBM355_
 
 int xshift_dirs(int stencil) { return stencil == LBM355_D2Q9 ? 6 : (stencil == LBM355_D3Q19 ? 10 : 18); }
 
-// LDS row shifting applies when a block can span a whole periodic row
+// LDS row shifting applies when a block can span a whole periodic row and rows are streamed (sweep_launch).
 // Not for FP16 storage: with 2-byte populations a wavefront access moves 128 bytes, and the barriers around the LDS
 // shift keep too few of them in flight.  The direct kernel, whose x-shifted loads are served partly from cache,
 // ran the D3Q27 cumulant AA-odd sweep at 256^3 in 0.441 ms against 0.487 ms on MI355X.  With both at their best
@@ -379,34 +379,35 @@ bool use_rowlds(const lbm355_sweep_desc* d, size_t* lds_bytes) {
 }
 
 // Dynamic LDS to request for a sweep launch: the kernel's own (kernel_lds), or more where a cap applies.
-size_t launch_lds(const lbm355_sweep_desc* d, bool rowlds, bool walls, size_t kernel_lds, unsigned block_threads) {
-  return lds_for_wave_cap(sweep_wave_cap(d, rowlds, walls, block_threads), block_threads, kernel_lds);
+size_t launch_lds(const lbm355_sweep_desc* d, const SweepLaunch& l, bool walls, size_t kernel_lds) {
+  const int cap = sweep_wave_cap(d, l.mode == ACCESS_ROWS, walls, l.half_cache, l.block.x);
+  return lds_for_wave_cap(cap, l.block.x, kernel_lds);
 }
 
 template <class TC>
-void* pick_kernel(const lbm355_sweep_desc* d, bool walls, bool rowlds) {
+void* pick_kernel(const lbm355_sweep_desc* d, bool walls, int mode) {
   constexpr bool f64 = sizeof(TC) == 8;
   const int st = d->stencil, sd = d->store_dtype, p = d->pattern;
   if (d->family == LBM355_FAMILY_MOMENT)
-    return f64 ? pick_sweep_moment_f64(st, sd, p, walls, rowlds) : pick_sweep_moment_f32(st, sd, p, walls, rowlds);
+    return f64 ? pick_sweep_moment_f64(st, sd, p, walls, mode) : pick_sweep_moment_f32(st, sd, p, walls, mode);
   if (d->family == LBM355_FAMILY_CENTRAL)
-    return f64 ? pick_sweep_central_f64(st, sd, p, walls, rowlds) : pick_sweep_central_f32(st, sd, p, walls, rowlds);
+    return f64 ? pick_sweep_central_f64(st, sd, p, walls, mode) : pick_sweep_central_f32(st, sd, p, walls, mode);
   if (d->family == LBM355_FAMILY_CUMULANT) {
     if (d->flags & LBM355_FLAG_LEARNED_CLOSURE)
       return f64 ? nullptr
                  : (d->flags & LBM355_FLAG_HIGHER_ORDERS_RATE1)
-                       ? pick_sweep_cumulant_learned_eq3_f32(st, sd, p, walls, rowlds)
-                       : pick_sweep_cumulant_learned_f32(st, sd, p, walls, rowlds);
+                       ? pick_sweep_cumulant_learned_eq3_f32(st, sd, p, walls, mode)
+                       : pick_sweep_cumulant_learned_f32(st, sd, p, walls, mode);
     if (d->flags & (LBM355_FLAG_GALILEAN | LBM355_FLAG_FOURTH_ORDER))
-      return f64 ? pick_sweep_cumulant_corrected_f64(st, sd, p, walls, rowlds)
-                 : pick_sweep_cumulant_corrected_f32(st, sd, p, walls, rowlds);
+      return f64 ? pick_sweep_cumulant_corrected_f64(st, sd, p, walls, mode)
+                 : pick_sweep_cumulant_corrected_f32(st, sd, p, walls, mode);
     if (d->flags & LBM355_FLAG_GENERAL_CUMULANT)
-      return f64 ? pick_sweep_cumulant_general_f64(st, sd, p, walls, rowlds)
-                 : pick_sweep_cumulant_general_f32(st, sd, p, walls, rowlds);
+      return f64 ? pick_sweep_cumulant_general_f64(st, sd, p, walls, mode)
+                 : pick_sweep_cumulant_general_f32(st, sd, p, walls, mode);
     if (d->flags & LBM355_FLAG_HIGHER_ORDERS_RATE1)
-      return f64 ? pick_sweep_cumulant_eq3_f64(st, sd, p, walls, rowlds)
-                 : pick_sweep_cumulant_eq3_f32(st, sd, p, walls, rowlds);
-    return f64 ? pick_sweep_cumulant_f64(st, sd, p, walls, rowlds) : pick_sweep_cumulant_f32(st, sd, p, walls, rowlds);
+      return f64 ? pick_sweep_cumulant_eq3_f64(st, sd, p, walls, mode)
+                 : pick_sweep_cumulant_eq3_f32(st, sd, p, walls, mode);
+    return f64 ? pick_sweep_cumulant_f64(st, sd, p, walls, mode) : pick_sweep_cumulant_f32(st, sd, p, walls, mode);
   }
   return nullptr;
 }
@@ -460,12 +461,13 @@ int launch_sweep(const lbm355_sweep_desc* d, const void* src, void* dst, void* r
   bool walls = false;
   for (int a = 0; a < stencil_d(d->stencil); ++a) walls |= d->face[a] == LBM355_FACE_NOSLIP;
   size_t lds = 0;
-  const bool rowlds = use_rowlds(d, &lds);
-  void* k = pick_kernel<TC>(d, walls, rowlds);
+  const bool odd = d->pattern == LBM355_AA_ODD;
+  const SweepLaunch l = sweep_launch(d, src, dst, use_rowlds(d, &lds), !odd, !odd);
+  void* k = pick_kernel<TC>(d, walls, l.mode);
   if (!k) return fail(LBM355_ERR_UNSUPPORTED, "no kernel for this stencil/family/dtype combination");
   SweepArgs<TC> a = make_args<TC>(d, src, dst, rho, u);
-  Launch l = geometry(d->nx, d->ny, d->nz, rowlds);
-  hipLaunchKernelGGL((KernelFn<TC>)k, l.grid, l.block, launch_lds(d, rowlds, walls, rowlds ? lds : 0, l.block.x), s, a);
+  a.order = l.order;
+  hipLaunchKernelGGL((KernelFn<TC>)k, l.grid, l.block, launch_lds(d, l, walls, l.mode == ACCESS_ROWS ? lds : 0), s, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(LBM355_ERR_LAUNCH, std::string("launch failed: ") + hipGetErrorString(e));
   return LBM355_OK;

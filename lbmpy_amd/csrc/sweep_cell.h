@@ -109,8 +109,8 @@ __host__ __device__ constexpr int n_xshift() {
 }
 
 // Non-temporal accesses for aligned, streamed-once data (each PDF is read and written exactly
-// once per sweep); misaligned (x +- 1) accesses keep the default policy so that the partially
-// used cache lines are served from cache to the neighbouring wavefront.
+// once per sweep); misaligned accesses (x +- 1, or all of them, see AccessMode) keep the default policy so that
+// the partially used cache lines are served from cache to the neighbouring wavefront.
 template <class TS, class TC>
 __device__ __forceinline__ TC load_nt(const TS* p) {
   return (TC)__builtin_nontemporal_load(p);
@@ -240,7 +240,8 @@ __device__ __forceinline__ void plane_store(TS* plane, int off, TC value) {
 // One cell of the sweep with direct (non-LDS) addressing: load with streaming, collide, store.
 // With WALLS, only cells next to a NoSlip face take the bounce-back addressing; the test is per cell and
 // the wall-free addressing is the same code as without WALLS, so interior cells pay nothing for walls.
-template <class S, int FAM, int PAT, bool WALLS, class TS, class TC>
+// NT: the accesses at the cell itself start on cache lines and are non-temporal.
+template <class S, int FAM, int PAT, bool WALLS, bool NT, class TS, class TC>
 __device__ __forceinline__ void sweep_cell(const SweepArgs<TC>& a, int x, int y, int z) {
   constexpr int Q = S::Q, D = S::D;
   const AxisNb ax = axis_neighbours(x, a.nx, a.g, a.face[0]);
@@ -263,20 +264,20 @@ __device__ __forceinline__ void sweep_cell(const SweepArgs<TC>& a, int x, int y,
   if constexpr (table_pattern(PAT)) {
     // Eso patterns and push: every access from the pattern's table (periodic wrap or ghost layer in X/Y/Z).
     // In place, a cell reads exactly the locations it writes, so one thread per cell needs no synchronisation.
-    // Accesses without an x offset are row-aligned and non-temporal.
+    // With NT, accesses without an x offset are row-aligned and non-temporal.
     constexpr AccessTable<S, PAT> acc{};
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
       const Access& t = acc.a[i];
       const TS* p = src + t.rslot * sq + X[1 + t.r[0]] + Y[1 + t.r[1]] + Z[1 + t.r[2]];
-      f[i] = t.r[0] == 0 ? load_nt<TS, TC>(p) : load_as<TS, TC>(p);
+      f[i] = NT && t.r[0] == 0 ? load_nt<TS, TC>(p) : load_as<TS, TC>(p);
     }
     collide_cell<S, FAM, TC, TS>(f, a, x, y, z);
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
       const Access& t = acc.a[i];
       TS* p = dst + t.wslot * sq + X[1 + t.w[0]] + Y[1 + t.w[1]] + Z[1 + t.w[2]];
-      if (t.w[0] == 0)
+      if (NT && t.w[0] == 0)
         store_nt<TS, TC>(p, f[i]);
       else
         store_as<TS, TC>(p, f[i]);
@@ -321,7 +322,7 @@ __device__ __forceinline__ void sweep_cell(const SweepArgs<TC>& a, int x, int y,
 
   if (PAT == LBM355_AA_EVEN) {
 #pragma unroll
-    for (int i = 0; i < Q; ++i) f[i] = plane_load<TS, TC, true>(src + i * sq, center);
+    for (int i = 0; i < Q; ++i) f[i] = plane_load<TS, TC, NT>(src + i * sq, center);
   } else if (near_wall) {
     load(std::true_type{});
   } else {
@@ -332,15 +333,111 @@ __device__ __forceinline__ void sweep_cell(const SweepArgs<TC>& a, int x, int y,
 
   if (PAT == LBM355_PULL) {
 #pragma unroll
-    for (int i = 0; i < Q; ++i) plane_store<TS, TC, true>(dst + i * sq, center, f[i]);
+    for (int i = 0; i < Q; ++i) plane_store<TS, TC, NT>(dst + i * sq, center, f[i]);
   } else if (PAT == LBM355_AA_EVEN) {
 #pragma unroll
-    for (int i = 0; i < Q; ++i) plane_store<TS, TC, true>(dst + S::inv[i] * sq, center, f[i]);
+    for (int i = 0; i < Q; ++i) plane_store<TS, TC, NT>(dst + S::inv[i] * sq, center, f[i]);
   } else if (near_wall) {
     store(std::true_type{});
   } else {
     store(std::false_type{});
   }
+}
+
+// How a sweep launch covers the cells and reaches memory:
+// ACCESS_ROWS    one block per whole periodic row, x-shifts through LDS, non-temporal accesses (the row kernels);
+// ACCESS_WAVES   one thread per cell, rows of whole wavefronts, accesses at the cell itself non-temporal;
+// ACCESS_LINES   the same with rows of any length, consecutive in memory;
+// ACCESS_CACHED  one thread per cell, regular accesses.
+enum AccessMode { ACCESS_ROWS, ACCESS_WAVES, ACCESS_LINES, ACCESS_CACHED };
+
+// The cell of this thread, or false beyond the last cell.  Threads number the cells consecutively over rows and
+// planes, so that wavefronts are full whatever nx is; with ACCESS_WAVES, blocks take up to 256 cells of one row, and y
+// and z stay in scalar registers (256^3 FP32 AA even: 593 us, 616 us with numbered cells; FP16 storage 315 and 329).
+template <int MODE, class TC>
+__device__ __forceinline__ bool thread_cell(const SweepArgs<TC>& a, int& x, int& y, int& z) {
+  if constexpr (MODE == ACCESS_WAVES) {
+    x = blockIdx.x * blockDim.x + threadIdx.x;
+    y = blockIdx.y;
+    z = blockIdx.z;
+    return x < a.nx;
+  }
+  const uint32_t t = a.order.number(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const uint32_t r = a.row.quotient(t), p = a.plane.quotient(r);
+  x = (int)(t - r * a.row.d);
+  y = (int)(r - p * a.plane.d);
+  z = (int)p;
+  return t < a.row.d * a.plane.d * (uint32_t)a.nz;
+}
+
+// Whether every wavefront's accesses at its own cells start on a 128-byte line, so that no two wavefronts share one:
+// the cells are consecutive in memory (no ghost layers, no padding), or rows are whole wavefronts on lines of their own.
+inline bool starts_lines(const lbm355_sweep_desc* d, const void* src, const void* dst) {
+  const int64_t es = d->store_dtype == LBM355_F64 ? 8 : (d->store_dtype == LBM355_F32 ? 4 : 2);
+  const bool flat = d->stencil == LBM355_D2Q9;
+  const int64_t first = d->ghost_layers * (1 + d->stride_y + (flat ? 0 : d->stride_z)) * es;
+  auto line = [](int64_t bytes) { return bytes % 128 == 0; };
+  if (!line((int64_t)(uintptr_t)src + first) || !line((int64_t)(uintptr_t)dst + first) || !line(d->stride_q * es))
+    return false;
+  if (d->ghost_layers == 0 && d->stride_y == d->nx && (flat || d->stride_z == (int64_t)d->nx * d->ny)) return true;
+  return d->nx % 64 == 0 && line(d->stride_y * es) && (flat || line(d->stride_z * es));
+}
+
+// Launch shape of a sweep, by what the populations' bytes (both arrays of a two-array pattern) fit into and how they lie.
+// Times on MI355X, us per launch before (row-mapped blocks, non-temporal accesses wherever x is unshifted) and now,
+// D3Q27 cumulant FP32 AA unless noted, every step on the same array:
+// - What fits the Infinity Cache (fits_cache) is found there by the next step, if it was written with regular stores:
+//   64^3 13.1 -> 10.0, 128^3 81.8 -> 56.7, 128^3 with ghost layers 145 -> 61, EsoTwist 100x90x80 28.2 -> 23.5, D3Q19 TRT
+//   pull 128x128x96 43.6 -> 33.0.  One run of blocks per XCD keeps a cell's neighbours in its L2 as well: D3Q19 SRT
+//   FP64 64x32x32 9.8 -> 7.4.  (The row kernel with regular accesses gave 61.2 at 128^3.)
+// - Above that, lines that start with a wavefront are best streamed past the caches, as they come: 256^3 593 (685 with
+//   regular accesses, 640 with runs of 16 blocks per XCD), FP16 250x200x180 252 -> 173.
+// - Otherwise two wavefronts share most lines, and non-temporal accesses move those twice; regular ones, with
+//   neighbouring blocks on one XCD, do not: 256^3 with ghost layers 947 -> 709 (809 without the runs), 251x255x253
+//   793 -> 684, FP64 131x117x101 143 -> 121.
+// Full wavefronts whatever nx is matter most for short rows: D3Q19 TRT 35x148x256 84 -> 31.
+constexpr uint32_t SHARED_LINES_CHUNK = 16;
+constexpr int64_t SMALL_CELLS = 1 << 18;   // below: blocks of one wavefront, to spread over the 256 CUs
+
+// Whether the populations' bytes fit the 256 MiB Infinity Cache to a gain.  In place in FP32 or FP64 they may fill it:
+// at 128^3 (216 MiB) regular accesses win also for a program that takes three such arrays in turn (82 -> 71 us, one
+// array 57).  Two arrays, FP16 storage and the learned closure lose more to such turns than they gain alone (pull D3Q19
+// 128x128x80, 253 MB: 36.7 -> 29.9 us for one pair of arrays, 42.5 for three in turn; FP16 192x128x128, 162 MiB: 54.7
+// -> 49.5, 63.5; closure 128^3: 107 -> 99, 116): they may fill half of it, where they do not (closure 128x96x96: 67 ->
+// 61, 66).
+inline int64_t population_bytes(const lbm355_sweep_desc* d, bool in_place) {
+  const int64_t es = d->store_dtype == LBM355_F64 ? 8 : (d->store_dtype == LBM355_F32 ? 4 : 2);
+  const int q = d->stencil == LBM355_D2Q9 ? 9 : (d->stencil == LBM355_D3Q19 ? 19 : 27);
+  return (in_place ? 1 : 2) * q * es * d->nx * d->ny * d->nz;
+}
+constexpr int64_t HALF_CACHE_BYTES = int64_t(128) << 20;
+inline bool fits_cache(const lbm355_sweep_desc* d, bool in_place) {
+  const bool half = !in_place || d->store_dtype == LBM355_F16 || (d->flags & LBM355_FLAG_LEARNED_CLOSURE);
+  return population_bytes(d, in_place) <= (half ? HALF_CACHE_BYTES : 2 * HALF_CACHE_BYTES);
+}
+
+struct SweepLaunch {
+  AccessMode mode;
+  dim3 grid, block;
+  XcdOrder order;
+  bool half_cache;   // the populations take at most HALF_CACHE_BYTES
+};
+
+// row_kernel, waves_kernel, lines_kernel: whether the caller has a kernel of that mode for this sweep.
+inline SweepLaunch sweep_launch(const lbm355_sweep_desc* d, const void* src, const void* dst, bool row_kernel,
+                                bool waves_kernel, bool lines_kernel) {
+  const bool fits = fits_cache(d, src == dst), half = population_bytes(d, src == dst) <= HALF_CACHE_BYTES;
+  const bool lines = !fits && starts_lines(d, src, dst);
+  if (row_kernel && lines) return {ACCESS_ROWS, dim3(1, d->ny, d->nz), dim3(d->nx), XcdOrder::of(1), half};
+  if (waves_kernel && lines && d->nx % 64 == 0) {
+    const unsigned bx = d->nx < 256 ? d->nx : 256;
+    return {ACCESS_WAVES, dim3((d->nx + bx - 1) / bx, d->ny, d->nz), dim3(bx), XcdOrder::of(1), half};
+  }
+  const int64_t cells = (int64_t)d->nx * d->ny * d->nz;
+  const unsigned bx = cells < SMALL_CELLS ? 64 : 256;
+  const unsigned blocks = (unsigned)((cells + bx - 1) / bx);
+  if (lines_kernel && lines) return {ACCESS_LINES, dim3(blocks), dim3(bx), XcdOrder::of(1), half};
+  return {ACCESS_CACHED, dim3(blocks), dim3(bx), XcdOrder::of(fits ? blocks / 8 : SHARED_LINES_CHUNK), half};
 }
 
 // Kernel arguments from a public descriptor (include/lbm355.h).
@@ -377,6 +474,9 @@ inline SweepArgs<TC> make_args(const lbm355_sweep_desc* d, const void* src, void
   a.u_in = (const TC*)d->velocity_in;
   a.nut_scale = (TC)(1.5 * d->smagorinsky_constant * d->smagorinsky_constant);
   a.seed = d->rounding_seed;
+  a.row = CellDivider::of((uint32_t)d->nx);
+  a.plane = CellDivider::of((uint32_t)d->ny);
+  a.order = XcdOrder::of(1);
   return a;
 }
 

@@ -5,17 +5,17 @@
 
 namespace lbm355 {
 
-void* pick_sweep_central_f64(int stencil, int store, int pat, bool walls, bool rowlds) {
-  if (stencil == LBM355_D2Q9) return pick_store<D2Q9, LBM355_FAMILY_CENTRAL, double>(store, pat, walls, rowlds);
-  if (stencil == LBM355_D3Q19) return pick_store<D3Q19, LBM355_FAMILY_CENTRAL, double>(store, pat, walls, rowlds);
-  if (stencil == LBM355_D3Q27) return pick_store<D3Q27, LBM355_FAMILY_CENTRAL, double>(store, pat, walls, rowlds);
+void* pick_sweep_central_f64(int stencil, int store, int pat, bool walls, int mode) {
+  if (stencil == LBM355_D2Q9) return pick_store<D2Q9, LBM355_FAMILY_CENTRAL, double>(store, pat, walls, mode);
+  if (stencil == LBM355_D3Q19) return pick_store<D3Q19, LBM355_FAMILY_CENTRAL, double>(store, pat, walls, mode);
+  if (stencil == LBM355_D3Q27) return pick_store<D3Q27, LBM355_FAMILY_CENTRAL, double>(store, pat, walls, mode);
   return nullptr;
 }
 
-void* eso_pick_central_f64(int stencil, int store, int pat, bool rows) {
-  if (stencil == LBM355_D2Q9) return eso_pick_store<D2Q9, LBM355_FAMILY_CENTRAL, double>(store, pat, rows);
-  if (stencil == LBM355_D3Q19) return eso_pick_store<D3Q19, LBM355_FAMILY_CENTRAL, double>(store, pat, rows);
-  if (stencil == LBM355_D3Q27) return eso_pick_store<D3Q27, LBM355_FAMILY_CENTRAL, double>(store, pat, rows);
+void* eso_pick_central_f64(int stencil, int store, int pat, int mode) {
+  if (stencil == LBM355_D2Q9) return eso_pick_store<D2Q9, LBM355_FAMILY_CENTRAL, double>(store, pat, mode);
+  if (stencil == LBM355_D3Q19) return eso_pick_store<D3Q19, LBM355_FAMILY_CENTRAL, double>(store, pat, mode);
+  if (stencil == LBM355_D3Q27) return eso_pick_store<D3Q27, LBM355_FAMILY_CENTRAL, double>(store, pat, mode);
   return nullptr;
 }
 

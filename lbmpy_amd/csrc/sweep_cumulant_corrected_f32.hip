@@ -5,14 +5,14 @@
 
 namespace lbm355 {
 
-void* pick_sweep_cumulant_corrected_f32(int stencil, int store, int pat, bool walls, bool rowlds) {
+void* pick_sweep_cumulant_corrected_f32(int stencil, int store, int pat, bool walls, int mode) {
   if (stencil != LBM355_D3Q27) return nullptr;
-  return pick_store<D3Q27, FAMILY_CUMULANT_CORRECTED, float>(store, pat, walls, rowlds);
+  return pick_store<D3Q27, FAMILY_CUMULANT_CORRECTED, float>(store, pat, walls, mode);
 }
 
-void* eso_pick_cumulant_corrected_f32(int stencil, int store, int pat, bool rows) {
+void* eso_pick_cumulant_corrected_f32(int stencil, int store, int pat, int mode) {
   if (stencil != LBM355_D3Q27) return nullptr;
-  return eso_pick_store<D3Q27, FAMILY_CUMULANT_CORRECTED, float>(store, pat, rows);
+  return eso_pick_store<D3Q27, FAMILY_CUMULANT_CORRECTED, float>(store, pat, mode);
 }
 
 }  // namespace lbm355

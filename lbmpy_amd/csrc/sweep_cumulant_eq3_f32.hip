@@ -6,14 +6,14 @@
 
 namespace lbm355 {
 
-void* pick_sweep_cumulant_eq3_f32(int stencil, int store, int pat, bool walls, bool rowlds) {
+void* pick_sweep_cumulant_eq3_f32(int stencil, int store, int pat, bool walls, int mode) {
   if (stencil != LBM355_D3Q27) return nullptr;
-  return pick_store<D3Q27, FAMILY_CUMULANT_EQ3, float>(store, pat, walls, rowlds);
+  return pick_store<D3Q27, FAMILY_CUMULANT_EQ3, float>(store, pat, walls, mode);
 }
 
-void* eso_pick_cumulant_eq3_f32(int stencil, int store, int pat, bool rows) {
+void* eso_pick_cumulant_eq3_f32(int stencil, int store, int pat, int mode) {
   if (stencil != LBM355_D3Q27) return nullptr;
-  return eso_pick_store<D3Q27, FAMILY_CUMULANT_EQ3, float>(store, pat, rows);
+  return eso_pick_store<D3Q27, FAMILY_CUMULANT_EQ3, float>(store, pat, mode);
 }
 
 }  // namespace lbm355

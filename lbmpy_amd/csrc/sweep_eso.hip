@@ -14,23 +14,23 @@
 namespace lbm355 {
 
 template <class TC>
-void* eso_pick(const lbm355_sweep_desc* d, bool rows) {
+void* eso_pick(const lbm355_sweep_desc* d, int mode) {
   constexpr bool f64 = sizeof(TC) == 8;
   const int sten = d->stencil, st = d->store_dtype, pat = d->pattern;
   if (d->family == LBM355_FAMILY_MOMENT)
-    return f64 ? eso_pick_moment_f64(sten, st, pat, rows) : eso_pick_moment_f32(sten, st, pat, rows);
+    return f64 ? eso_pick_moment_f64(sten, st, pat, mode) : eso_pick_moment_f32(sten, st, pat, mode);
   if (d->family == LBM355_FAMILY_CENTRAL)
-    return f64 ? eso_pick_central_f64(sten, st, pat, rows) : eso_pick_central_f32(sten, st, pat, rows);
+    return f64 ? eso_pick_central_f64(sten, st, pat, mode) : eso_pick_central_f32(sten, st, pat, mode);
   if (d->family == LBM355_FAMILY_CUMULANT) {
     if (d->flags & (LBM355_FLAG_GALILEAN | LBM355_FLAG_FOURTH_ORDER))
-      return f64 ? eso_pick_cumulant_corrected_f64(sten, st, pat, rows)
-                 : eso_pick_cumulant_corrected_f32(sten, st, pat, rows);
+      return f64 ? eso_pick_cumulant_corrected_f64(sten, st, pat, mode)
+                 : eso_pick_cumulant_corrected_f32(sten, st, pat, mode);
     if (d->flags & LBM355_FLAG_GENERAL_CUMULANT)
-      return f64 ? eso_pick_cumulant_general_f64(sten, st, pat, rows)
-                 : eso_pick_cumulant_general_f32(sten, st, pat, rows);
+      return f64 ? eso_pick_cumulant_general_f64(sten, st, pat, mode)
+                 : eso_pick_cumulant_general_f32(sten, st, pat, mode);
     if (d->flags & LBM355_FLAG_HIGHER_ORDERS_RATE1)
-      return f64 ? eso_pick_cumulant_eq3_f64(sten, st, pat, rows) : eso_pick_cumulant_eq3_f32(sten, st, pat, rows);
-    return f64 ? eso_pick_cumulant_f64(sten, st, pat, rows) : eso_pick_cumulant_f32(sten, st, pat, rows);
+      return f64 ? eso_pick_cumulant_eq3_f64(sten, st, pat, mode) : eso_pick_cumulant_eq3_f32(sten, st, pat, mode);
+    return f64 ? eso_pick_cumulant_f64(sten, st, pat, mode) : eso_pick_cumulant_f32(sten, st, pat, mode);
   }
   return nullptr;
 }
@@ -46,18 +46,21 @@ int lbm355_launch_sweep_eso(const lbm355_sweep_desc* d, const void* src, void* d
   const int rows_needed = d->stencil == LBM355_D2Q9 ? eso_max_rows<D2Q9>()
                           : d->stencil == LBM355_D3Q19 ? eso_max_rows<D3Q19>() : eso_max_rows<D3Q27>();
   const size_t lds = (size_t)rows_needed * d->nx * es;
-  const bool rows = d->face[0] == LBM355_FACE_PERIODIC && d->nx % 64 == 0 && d->nx <= 512 && lds <= 65536;
-  void* k = d->compute_dtype == LBM355_F64 ? eso_pick<double>(d, rows) : eso_pick<float>(d, rows);
+  const bool row_kernel = d->face[0] == LBM355_FACE_PERIODIC && d->nx % 64 == 0 && d->nx <= 512 && lds <= 65536;
+  // the rows that a cell reaches beside its own start on lines, too, only if rows are whole wavefronts
+  const SweepLaunch l = sweep_launch(d, src, dst, row_kernel, true, false);
+  const bool rows = l.mode == ACCESS_ROWS;
+  void* k = d->compute_dtype == LBM355_F64 ? eso_pick<double>(d, l.mode) : eso_pick<float>(d, l.mode);
   if (!k) return lbm355_set_error(LBM355_ERR_UNSUPPORTED, "no Eso kernel for this stencil/family/dtype combination");
-  const int bx = rows ? d->nx : (d->nx >= 256 ? 256 : ((d->nx + 63) / 64) * 64);
-  const dim3 grid((d->nx + bx - 1) / bx, d->ny, d->nz), block(bx);
-  const size_t shm = lds_for_wave_cap(sweep_wave_cap(d, rows, false, bx), bx, rows ? lds : 0);
+  const size_t shm = lds_for_wave_cap(sweep_wave_cap(d, rows, false, l.half_cache, l.block.x), l.block.x, rows ? lds : 0);
   if (d->compute_dtype == LBM355_F64) {
     SweepArgs<double> a = make_args<double>(d, src, dst, rho, u);
-    hipLaunchKernelGGL((void (*)(SweepArgs<double>))k, grid, block, shm, s, a);
+    a.order = l.order;
+    hipLaunchKernelGGL((void (*)(SweepArgs<double>))k, l.grid, l.block, shm, s, a);
   } else {
     SweepArgs<float> a = make_args<float>(d, src, dst, rho, u);
-    hipLaunchKernelGGL((void (*)(SweepArgs<float>))k, grid, block, shm, s, a);
+    a.order = l.order;
+    hipLaunchKernelGGL((void (*)(SweepArgs<float>))k, l.grid, l.block, shm, s, a);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess)

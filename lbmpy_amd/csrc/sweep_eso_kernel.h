@@ -6,11 +6,11 @@
 
 namespace lbm355 {
 
-template <class S, int FAM, int PAT, class TS, class TC>
+template <class S, int FAM, int PAT, int MODE, class TS, class TC>
 __global__ void __launch_bounds__(256) sweep_eso_kernel(SweepArgs<TC> a) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= a.nx) return;
-  sweep_cell<S, FAM, PAT, false, TS, TC>(a, x, blockIdx.y, blockIdx.z);
+  int x, y, z;
+  if (!thread_cell<MODE>(a, x, y, z)) return;
+  sweep_cell<S, FAM, PAT, false, MODE != ACCESS_CACHED, TS, TC>(a, x, y, z);
 }
 
 // x-shifted accesses of the table (compile-time counts, for the LDS rows of the row-staged kernel)
@@ -131,35 +131,39 @@ constexpr int eso_max_rows() {
   return m;
 }
 
-template <class S, int FAM, class TS, class TC>
+template <class S, int FAM, int MODE, class TS, class TC>
 void* eso_pick_pattern(int pat) {
   switch (pat) {
-    case LBM355_ESOTWIST_EVEN: return (void*)sweep_eso_kernel<S, FAM, LBM355_ESOTWIST_EVEN, TS, TC>;
-    case LBM355_ESOTWIST_ODD: return (void*)sweep_eso_kernel<S, FAM, LBM355_ESOTWIST_ODD, TS, TC>;
-    case LBM355_ESOPULL_EVEN: return (void*)sweep_eso_kernel<S, FAM, LBM355_ESOPULL_EVEN, TS, TC>;
-    case LBM355_ESOPULL_ODD: return (void*)sweep_eso_kernel<S, FAM, LBM355_ESOPULL_ODD, TS, TC>;
-    case LBM355_ESOPUSH_EVEN: return (void*)sweep_eso_kernel<S, FAM, LBM355_ESOPUSH_EVEN, TS, TC>;
-    case LBM355_ESOPUSH_ODD: return (void*)sweep_eso_kernel<S, FAM, LBM355_ESOPUSH_ODD, TS, TC>;
-    case LBM355_PUSH: return (void*)sweep_eso_kernel<S, FAM, LBM355_PUSH, TS, TC>;
+    case LBM355_ESOTWIST_EVEN: return (void*)sweep_eso_kernel<S, FAM, LBM355_ESOTWIST_EVEN, MODE, TS, TC>;
+    case LBM355_ESOTWIST_ODD: return (void*)sweep_eso_kernel<S, FAM, LBM355_ESOTWIST_ODD, MODE, TS, TC>;
+    case LBM355_ESOPULL_EVEN: return (void*)sweep_eso_kernel<S, FAM, LBM355_ESOPULL_EVEN, MODE, TS, TC>;
+    case LBM355_ESOPULL_ODD: return (void*)sweep_eso_kernel<S, FAM, LBM355_ESOPULL_ODD, MODE, TS, TC>;
+    case LBM355_ESOPUSH_EVEN: return (void*)sweep_eso_kernel<S, FAM, LBM355_ESOPUSH_EVEN, MODE, TS, TC>;
+    case LBM355_ESOPUSH_ODD: return (void*)sweep_eso_kernel<S, FAM, LBM355_ESOPUSH_ODD, MODE, TS, TC>;
+    case LBM355_PUSH: return (void*)sweep_eso_kernel<S, FAM, LBM355_PUSH, MODE, TS, TC>;
   }
   return nullptr;
 }
 
+template <class S, int FAM, class TS, class TC>
+void* eso_pick_mode(int pat, int mode) {
+  if (mode == ACCESS_ROWS) return eso_pick_rows<S, FAM, TS, TC>(pat);
+  return mode == ACCESS_WAVES ? eso_pick_pattern<S, FAM, ACCESS_WAVES, TS, TC>(pat)
+                              : eso_pick_pattern<S, FAM, ACCESS_CACHED, TS, TC>(pat);
+}
+
 template <class S, int FAM, class TC>
-void* eso_pick_store(int store, int pat, bool rows) {
-  if (store == LBM355_F64)
-    return rows ? eso_pick_rows<S, FAM, double, TC>(pat) : eso_pick_pattern<S, FAM, double, TC>(pat);
-  if (store == LBM355_F32)
-    return rows ? eso_pick_rows<S, FAM, float, TC>(pat) : eso_pick_pattern<S, FAM, float, TC>(pat);
+void* eso_pick_store(int store, int pat, int mode) {
+  if (store == LBM355_F64) return eso_pick_mode<S, FAM, double, TC>(pat, mode);
+  if (store == LBM355_F32) return eso_pick_mode<S, FAM, float, TC>(pat, mode);
   if constexpr (sizeof(TC) == 4) {
-    if (store == LBM355_F16)
-      return rows ? eso_pick_rows<S, FAM, _Float16, TC>(pat) : eso_pick_pattern<S, FAM, _Float16, TC>(pat);
+    if (store == LBM355_F16) return eso_pick_mode<S, FAM, _Float16, TC>(pat, mode);
   }
   return nullptr;
 }
 
 // Eso / push kernel pickers of each (family, compute type), one per translation unit; NULL when there is none.
-#define LBM355_ESO_PICKER(NAME) void* NAME(int stencil, int store, int pat, bool rows)
+#define LBM355_ESO_PICKER(NAME) void* NAME(int stencil, int store, int pat, int mode)
 LBM355_ESO_PICKER(eso_pick_moment_f64);
 LBM355_ESO_PICKER(eso_pick_moment_f32);
 LBM355_ESO_PICKER(eso_pick_central_f64);

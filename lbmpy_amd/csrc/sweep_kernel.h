@@ -8,13 +8,14 @@
 
 namespace lbm355 {
 
-template <class S, int FAM, int PAT, bool WALLS, bool ROWLDS, class TS, class TC>
-__global__ void __launch_bounds__(ROWLDS ? 512 : 256) sweep_kernel(SweepArgs<TC> a) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
-  if constexpr (!ROWLDS) {
-    if (x >= a.nx) return;
-    sweep_cell<S, FAM, PAT, WALLS, TS, TC>(a, x, blockIdx.y, blockIdx.z);
+template <class S, int FAM, int PAT, bool WALLS, int MODE, class TS, class TC>
+__global__ void __launch_bounds__(MODE == ACCESS_ROWS ? 512 : 256) sweep_kernel(SweepArgs<TC> a) {
+  if constexpr (MODE != ACCESS_ROWS) {
+    int x, y, z;
+    if (!thread_cell<MODE>(a, x, y, z)) return;
+    sweep_cell<S, FAM, PAT, WALLS, MODE != ACCESS_CACHED, TS, TC>(a, x, y, z);
   } else {
+    const int x = blockIdx.x * blockDim.x + threadIdx.x;
     // The block spans one whole periodic row (blockDim.x == nx).  The +-1 x-shifts of pull / AA-odd
     // streaming go through LDS, so every global access is an aligned, contiguous, non-temporal one.
     constexpr int Q = S::Q, D = S::D;
@@ -119,10 +120,7 @@ __global__ void __launch_bounds__(ROWLDS ? 512 : 256) sweep_kernel(SweepArgs<TC>
       }
     };
 
-    if (PAT == LBM355_AA_EVEN) {
-#pragma unroll
-      for (int i = 0; i < Q; ++i) f[i] = load_nt<TS, TC>(src + i * sq + center);
-    } else if (row_walls) {
+    if (row_walls) {
       load(std::true_type{});
     } else {
       load(std::false_type{});
@@ -133,9 +131,6 @@ __global__ void __launch_bounds__(ROWLDS ? 512 : 256) sweep_kernel(SweepArgs<TC>
     if (PAT == LBM355_PULL) {
 #pragma unroll
       for (int i = 0; i < Q; ++i) store_nt<TS, TC>(dst + i * sq + center, f[i]);
-    } else if (PAT == LBM355_AA_EVEN) {
-#pragma unroll
-      for (int i = 0; i < Q; ++i) store_nt<TS, TC>(dst + S::inv[i] * sq + center, f[i]);
     } else if (row_walls) {
       store(std::true_type{});
     } else {
@@ -144,35 +139,42 @@ __global__ void __launch_bounds__(ROWLDS ? 512 : 256) sweep_kernel(SweepArgs<TC>
   }
 }
 
-template <class S, int FAM, class TS, class TC>
-void* pick_pattern(int pat, bool walls, bool rowlds) {
-#define LBM_K(P, W, R) (void*)sweep_kernel<S, FAM, P, W, R, TS, TC>
-  switch (pat) {
-    case LBM355_PULL:
-      if (rowlds) return walls ? LBM_K(LBM355_PULL, true, true) : LBM_K(LBM355_PULL, false, true);
-      return walls ? LBM_K(LBM355_PULL, true, false) : LBM_K(LBM355_PULL, false, false);
-    case LBM355_AA_EVEN:
-      return LBM_K(LBM355_AA_EVEN, false, false);
-    case LBM355_AA_ODD:
-      if (rowlds) return walls ? LBM_K(LBM355_AA_ODD, true, true) : LBM_K(LBM355_AA_ODD, false, true);
-      return walls ? LBM_K(LBM355_AA_ODD, true, false) : LBM_K(LBM355_AA_ODD, false, false);
+// AA even has no x-shifts (no row kernel); AA odd reaches no population but the centre's at the cell itself, so its
+// per-cell kernel is the ACCESS_CACHED one.
+template <class S, int FAM, bool WALLS, class TS, class TC>
+void* pick_walls(int pat, int mode) {
+#define LBM_K(P, M) (void*)sweep_kernel<S, FAM, P, WALLS, M, TS, TC>
+  if (pat == LBM355_PULL) {
+    if (mode == ACCESS_ROWS) return LBM_K(LBM355_PULL, ACCESS_ROWS);
+    if (mode == ACCESS_WAVES) return LBM_K(LBM355_PULL, ACCESS_WAVES);
+    return mode == ACCESS_LINES ? LBM_K(LBM355_PULL, ACCESS_LINES) : LBM_K(LBM355_PULL, ACCESS_CACHED);
   }
-#undef LBM_K
+  if (pat == LBM355_AA_ODD) return mode == ACCESS_ROWS ? LBM_K(LBM355_AA_ODD, ACCESS_ROWS) : LBM_K(LBM355_AA_ODD, ACCESS_CACHED);
   return nullptr;
+#undef LBM_K
+}
+
+template <class S, int FAM, class TS, class TC>
+void* pick_pattern(int pat, bool walls, int mode) {
+#define LBM_K(M) (void*)sweep_kernel<S, FAM, LBM355_AA_EVEN, false, M, TS, TC>
+  if (pat == LBM355_AA_EVEN)
+    return mode == ACCESS_WAVES ? LBM_K(ACCESS_WAVES) : mode == ACCESS_LINES ? LBM_K(ACCESS_LINES) : LBM_K(ACCESS_CACHED);
+#undef LBM_K
+  return walls ? pick_walls<S, FAM, true, TS, TC>(pat, mode) : pick_walls<S, FAM, false, TS, TC>(pat, mode);
 }
 
 template <class S, int FAM, class TC>
-void* pick_store(int store, int pat, bool walls, bool rowlds) {
-  if (store == LBM355_F64) return pick_pattern<S, FAM, double, TC>(pat, walls, rowlds);
-  if (store == LBM355_F32) return pick_pattern<S, FAM, float, TC>(pat, walls, rowlds);
+void* pick_store(int store, int pat, bool walls, int mode) {
+  if (store == LBM355_F64) return pick_pattern<S, FAM, double, TC>(pat, walls, mode);
+  if (store == LBM355_F32) return pick_pattern<S, FAM, float, TC>(pat, walls, mode);
   if constexpr (sizeof(TC) == 4) {
-    if (store == LBM355_F16) return pick_pattern<S, FAM, _Float16, TC>(pat, walls, rowlds);
+    if (store == LBM355_F16) return pick_pattern<S, FAM, _Float16, TC>(pat, walls, mode);
   }
   return nullptr;
 }
 
 // Kernel pickers of each (family, compute type), one per translation unit; NULL when there is no kernel.
-#define LBM355_PICKER(NAME) void* NAME(int stencil, int store, int pat, bool walls, bool rowlds)
+#define LBM355_PICKER(NAME) void* NAME(int stencil, int store, int pat, bool walls, int mode)
 LBM355_PICKER(pick_sweep_moment_f64);
 LBM355_PICKER(pick_sweep_moment_f32);
 LBM355_PICKER(pick_sweep_central_f64);
