@@ -362,9 +362,25 @@ int lbm355_closure_features(const float* pi_neq, const float* density, int64_t n
 int lbm355_closure_forward(const void* params, const float* features, int64_t n, float* out, void* stream);
 
 /* gradient of L = (1/n) sum (softplus(o) - targets)^2 into grad[master_size] (overwritten), L into
- * loss[0]; `blocks` persistent one-wavefront blocks. */
+ * loss[0], by atomic sums; `blocks` persistent wavefronts. */
 int lbm355_closure_train_step(const void* params, const float* features, const float* targets, int64_t n,
                               float* grad, float* loss, int32_t blocks, void* stream);
+
+/* Floats of the device workspace of the two functions below (per-block sums; overwritten). */
+int64_t lbm355_closure_workspace_floats(void);
+
+/* The same gradient and loss, summed in a fixed order through `workspace`. */
+int lbm355_closure_gradient(const void* params, const float* features, const float* targets, int64_t n, float* grad,
+                            float* loss, float* workspace, void* stream);
+
+/* One epoch of Adam on minibatches of up to `batch` samples, taken in the order of the device array order[n] (row
+ * indices into features and targets): per minibatch the gradient at the current parameters and one Adam step, as
+ * lbm355_closure_gradient and lbm355_closure_adam (with step = steps_done + 1, ...) compute them.  losses[k]: the
+ * k-th minibatch's loss, ceil(n / batch) of them. */
+int lbm355_closure_train_epoch(void* params, float* master, float* m, float* v, const float* features,
+                               const float* targets, const int64_t* order, int64_t n, int64_t batch, float lr,
+                               float beta1, float beta2, float eps, int32_t steps_done, float* losses, float* workspace,
+                               void* stream);
 
 /* Adam step (`step` >= 1) on the FP32 master parameters with moments m, v; re-packs the BF16
  * weights and FP32 biases into the parameter block `params`. */

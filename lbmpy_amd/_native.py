@@ -64,7 +64,8 @@ EXPORTED = ("lbm355_sweep", "lbm355_table_elements", "lbm355_noslip_links", "lbm
             "lbm355_last_error", "lbm355_version", "lbm355_batch_create", "lbm355_batch_sweep",
             "lbm355_batch_info", "lbm355_batch_destroy", "lbm355_batch_sweep_static", "lbm355_closure_params_size",
             "lbm355_closure_master_size", "lbm355_closure_features", "lbm355_closure_forward",
-            "lbm355_closure_train_step", "lbm355_closure_adam", "lbm355_boundary_links", "lbm355_copy_boxes",
+            "lbm355_closure_train_step", "lbm355_closure_adam", "lbm355_closure_workspace_floats",
+            "lbm355_closure_gradient", "lbm355_closure_train_epoch", "lbm355_boundary_links", "lbm355_copy_boxes",
             "lbm355_pattern_access", "lbm355_get_strain_rate", "lbm355_plane_copy", "lbm355_valu_probe",
             "lbm355_source_hash")
 
@@ -129,6 +130,14 @@ def load(path=None):
     lib.lbm355_closure_adam.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, ctypes.c_float, ctypes.c_float,
                                         ctypes.c_float, ctypes.c_float, c_int32, c_void_p, c_void_p]
     lib.lbm355_closure_adam.restype = c_int32
+    lib.lbm355_closure_workspace_floats.argtypes = []
+    lib.lbm355_closure_workspace_floats.restype = c_int64
+    lib.lbm355_closure_gradient.argtypes = [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p,
+                                            c_void_p]
+    lib.lbm355_closure_gradient.restype = c_int32
+    lib.lbm355_closure_train_epoch.argtypes = [c_void_p] * 7 + [c_int64, c_int64] + [ctypes.c_float] * 4 + \
+        [c_int32, c_void_p, c_void_p, c_void_p]
+    lib.lbm355_closure_train_epoch.restype = c_int32
     lib.lbm355_boundary_links.argtypes = [ctypes.POINTER(BoundaryDesc), c_void_p, c_void_p, c_int64, c_void_p,
                                           c_void_p]
     lib.lbm355_boundary_links.restype = c_int32

@@ -134,14 +134,20 @@ class ClosureModel:
         return self.nu_scale * torch.nn.functional.softplus(self.forward(features))
 
     def gradient(self, features, targets, blocks=1024):
-        """(loss, grad) of L = mean((softplus(o) - y)^2) at the current parameters (GPU kernels)."""
+        """(loss, grad) of L = mean((softplus(o) - y)^2) at the current parameters (GPU kernels).  `blocks` has no
+        effect: the sums' order is fixed."""
         x = features.float().contiguous()
         y = targets.float().contiguous()
         grad = torch.empty(MASTER_SIZE, dtype=torch.float32, device=self.device)
         loss = torch.empty(1, dtype=torch.float32, device=self.device)
-        nat.check(self.lib.lbm355_closure_train_step(_ptr(self.params), _ptr(x), _ptr(y), x.shape[0], _ptr(grad),
-                                                     _ptr(loss), blocks, nat.current_stream_handle()))
+        if blocks <= 0:
+            raise nat.LbmError("closure gradient: blocks must be positive")
+        nat.check(self.lib.lbm355_closure_gradient(_ptr(self.params), _ptr(x), _ptr(y), x.shape[0], _ptr(grad),
+                                                   _ptr(loss), _ptr(self._workspace()), nat.current_stream_handle()))
         return loss, grad
+
+    def _workspace(self):
+        return torch.empty(self.lib.lbm355_closure_workspace_floats(), dtype=torch.float32, device=self.device)
 
     def adam_step(self, grad, lr=1e-3, beta1=0.9, beta2=0.999, eps=1e-8):
         self.step += 1
@@ -151,19 +157,25 @@ class ClosureModel:
     def train(self, features, targets, epochs=4, batch=65536, lr=2e-3, seed=0, log=None):
         """Adam on minibatches of (features, targets = nu_t / nu_scale); returns the per-epoch mean loss."""
         n = features.shape[0]
+        x = features.float().contiguous()
+        y = targets.float().contiguous()
+        if not (x.is_cuda and y.is_cuda) or x.numel() != n * IN or y.numel() < n:
+            raise ValueError(f"training takes GPU tensors of features ({n}, {IN}) and {n} targets, not "
+                             f"{tuple(x.shape)} on {x.device} and {tuple(y.shape)} on {y.device}")
+        workspace = self._workspace()
+        losses = torch.empty(len(range(0, n, batch)), dtype=torch.float32, device=self.device)
+        nb = len(losses)
         g = torch.Generator(device=self.device).manual_seed(seed)
         history = []
         for ep in range(epochs):
             perm = torch.randperm(n, generator=g, device=self.device)
-            tot = torch.zeros((), device=self.device, dtype=torch.float64)
-            nb = 0
-            for s in range(0, n, batch):
-                idx = perm[s:s + batch]
-                loss, grad = self.gradient(features[idx], targets[idx])
-                self.adam_step(grad, lr=lr)
-                tot += loss[0].double()
-                nb += 1
-            history.append(float(tot / nb))
+            if nb:
+                nat.check(self.lib.lbm355_closure_train_epoch(
+                    _ptr(self.params), _ptr(self.master), _ptr(self.m), _ptr(self.v), _ptr(x), _ptr(y), _ptr(perm), n,
+                    batch, lr, 0.9, 0.999, 1e-8, self.step, _ptr(losses), _ptr(workspace),
+                    nat.current_stream_handle()))
+                self.step += nb
+            history.append(float(losses.double().sum() / nb))
             if log:
                 log(f"closure training epoch {ep}: loss {history[-1]:.4e}")
         return history
