@@ -27,6 +27,9 @@ HIP_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
     # no packed FP32 instructions (v_pk_*_f32): keep arithmetic on the plain VALU path
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # matrix products write vector registers where the registers allow it: results in accumulation registers take one
+    # more instruction each to be read (64 of 1,750 in the learned-closure sweep)
+    "-mllvm", "-amdgpu-mfma-vgpr-form=1",
     "-ffp-contract=fast", "-munsafe-fp-atomics",
     "-Wno-unused-result",
 ]

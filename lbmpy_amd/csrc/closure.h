@@ -20,6 +20,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "lbm_common.h"
+
 namespace lbm355 {
 
 constexpr int CLOSURE_IN = 10, CLOSURE_IN_PAD = 16, CLOSURE_H = 32;
@@ -51,7 +53,7 @@ __device__ __forceinline__ float sigmoid(float o) { return 1.f / (1.f + expf(-o)
 
 // raw features from the non-equilibrium second moments Pi_neq (xx, yy, zz, xy, xz, yz) and rho
 __device__ __forceinline__ void closure_features(const float (&p)[6], float rho, float (&x)[CLOSURE_IN]) {
-  const float ir = 1.f / rho;
+  const float ir = recip(rho);
   const float q[6] = {p[0] * ir, p[1] * ir, p[2] * ir, p[3] * ir, p[4] * ir, p[5] * ir};
   const float qq = q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + 2.f * (q[3] * q[3] + q[4] * q[4] + q[5] * q[5]);
   // tr(q^3) of the symmetric matrix [[xx, xy, xz], [xy, yy, yz], [xz, yz, zz]]
@@ -60,17 +62,24 @@ __device__ __forceinline__ void closure_features(const float (&p)[6], float rho,
                    6.f * q[3] * q[4] * q[5];
 #pragma unroll
   for (int i = 0; i < 6; ++i) x[i] = q[i];
-  x[6] = sqrtf(2.f * qq);
+  x[6] = __builtin_amdgcn_sqrtf(2.f * qq);
   x[7] = q[0] + q[1] + q[2];
   x[8] = qq;
   x[9] = t3;
 }
 
-// tanh in FP32 for the hidden layers: sign(x) (1 - e) / (1 + e) with e = exp(-2|x|) from the hardware base-2
-// exponential and reciprocal; absolute error about 2e-7, far below the BF16 step of the activations that the
-// next layer reads.  Five plain instructions and two transcendental ones, no select.
+// tanh in FP32 for the hidden layers: 1 - 2 / (1 + e) with e = exp(2x) from the hardware base-2 exponential and
+// reciprocal (e = inf and 0 give +-1); absolute error about 2e-7, far below the BF16 step of the activations that the
+// next layer reads.  Three plain instructions and two transcendental ones; each cell takes 64 of them.
 __device__ __forceinline__ float tanh_fast(float x) {
-  const float e = __builtin_amdgcn_exp2f(-2.885390081777927f * fabsf(x));   // 2 log2(e) |x|
+  const float e = __builtin_amdgcn_exp2f(2.885390081777927f * x);   // 2 log2(e) x
+  return __builtin_fmaf(-2.f, __builtin_amdgcn_rcpf(1.f + e), 1.f);
+}
+
+// The same as an exactly odd function, sign(x) (1 - e) / (1 + e) with e = exp(-2|x|): two instructions more, which
+// training, bound by latency, does not notice.
+__device__ __forceinline__ float tanh_odd(float x) {
+  const float e = __builtin_amdgcn_exp2f(-2.885390081777927f * fabsf(x));
   return copysignf((1.f - e) * __builtin_amdgcn_rcpf(1.f + e), x);
 }
 
@@ -92,6 +101,7 @@ __device__ __forceinline__ int c_row(int v, int lane) { return 8 * (v >> 2) + 4 
 // Wave-collective forward pass for the 64 cells of a wavefront (every lane must take part).
 // x: this lane's raw features.  Returns this lane's output o.  If h1/h2 are given, the tanh
 // activations of both cell blocks c = 0, 1 are kept in C layout (h[c][v]) for the backward pass.
+template <bool TRAINING = false>
 __device__ __forceinline__ float mlp_forward_wave(const ClosureParams* __restrict__ P, const float (&x)[CLOSURE_IN],
                                                   float (*h1)[16], float (*h2)[16]) {
   const int lane = threadIdx.x & 63;
@@ -137,7 +147,7 @@ __device__ __forceinline__ float mlp_forward_wave(const ClosureParams* __restric
     v4s hb[4];
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      const float h = tanh_fast(acc[v]);
+      const float h = TRAINING ? tanh_odd(acc[v]) : tanh_fast(acc[v]);
       if (h1) h1[c][v] = h;
       hb[v >> 2][v & 3] = (short)f2bf(h);
     }
@@ -149,7 +159,7 @@ __device__ __forceinline__ float mlp_forward_wave(const ClosureParams* __restric
     float part = 0.f;
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      const float h = tanh_fast(acc2[v]);
+      const float h = TRAINING ? tanh_odd(acc2[v]) : tanh_fast(acc2[v]);
       if (h2) h2[c][v] = h;
       part += bf2f(P->w3[c_row(v, lane)]) * h;
     }
@@ -162,8 +172,12 @@ __device__ __forceinline__ float mlp_forward_wave(const ClosureParams* __restric
 // shear relaxation rate from the network output: nu_t = nu_scale softplus(o) - nu_shift added to the
 // molecular viscosity, relaxation time at least 0.5 + 3e-6
 __device__ __forceinline__ float closure_omega(const ClosureParams* __restrict__ P, float o, float omega0) {
-  const float tau = 1.f / omega0 + 3.f * (P->nu_scale * softplus(o) - P->nu_shift);
-  return 1.f / fmaxf(tau, 0.500003f);
+  // softplus(o) = max(o, 0) + log(1 + exp(-|o|)) with the hardware's base-2 functions: absolute error below 2e-7, which
+  // nu_scale makes small against the rounding of tau
+  const float e = __builtin_amdgcn_exp2f(-1.4426950408889634f * fabsf(o));
+  const float sp = __builtin_fmaf(0.6931471805599453f, __builtin_amdgcn_logf(1.f + e), fmaxf(o, 0.f));
+  const float tau = recip(omega0) + 3.f * (P->nu_scale * sp - P->nu_shift);
+  return recip(fmaxf(tau, 0.500003f));
 }
 
 }  // namespace lbm355

@@ -115,7 +115,7 @@ __global__ void __launch_bounds__(64 * TRAIN_WAVES) train_kernel(const ClosurePa
     for (int k = 0; k < CLOSURE_IN; ++k) x[k] = valid ? X[CLOSURE_IN * row + k] : 0.f;
     const float y = valid ? Y[row] : 0.f;
     float h1[2][16], h2[2][16];
-    const float o = mlp_forward_wave(P, x, h1, h2);
+    const float o = mlp_forward_wave<true>(P, x, h1, h2);
     const float diff = softplus(o) - y;
     const float g = valid ? 2.f * inv_n * diff * sigmoid(o) : 0.f;
     lsum += valid ? diff * diff : 0.f;
