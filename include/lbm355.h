@@ -208,6 +208,19 @@ int lbm355_set_equilibrium(const lbm355_sweep_desc* desc, void* pdf, const doubl
 int lbm355_get_macroscopic(const lbm355_sweep_desc* desc, const void* pdf, double* density, double* velocity,
                            int32_t last_pattern, void* stream);
 
+/* The same into fields of either type and any order: element (x, y, z, c) of the interior at x stride[0] + y stride[1] +
+ * z stride[2] + c vector_stride[3] elements from the field's pointer (2-D: no z).  density_deviation is density - 1.
+ * NULL leaves a field out.  The pointers may be pinned host memory. */
+typedef struct lbm355_macroscopic_out {
+  void *density, *density_deviation, *velocity;
+  int64_t scalar_stride[3];   /* density, density_deviation */
+  int64_t vector_stride[4];   /* velocity */
+  int32_t dtype, pad;         /* LBM355_F64 or LBM355_F32 */
+} lbm355_macroscopic_out;
+
+int lbm355_get_fields(const lbm355_sweep_desc* desc, const void* pdf, const lbm355_macroscopic_out* out,
+                      int32_t last_pattern, void* stream);
+
 /* Strain-rate tensor S_ab = -1.5 (omega_shear / rho_ref) sum_i c_ia c_ib (f_i - f_eq,i(rho, u)) of the populations
  * the kernel `last_pattern` wrote (read as lbm355_get_macroscopic reads them; rho and the equilibrium velocity u
  * as the collision computes them, rho_ref = rho if compressible, else 1): lbmpy's strain_rate_tensor_getter

@@ -58,9 +58,14 @@ class SweepDesc(ctypes.Structure):
                 ("velocity_in", c_void_p), ("rounding_seed", ctypes.c_uint32), ("waves_per_simd", c_int32)]
 
 
+class MacroscopicOut(ctypes.Structure):
+    _fields_ = [("density", c_void_p), ("density_deviation", c_void_p), ("velocity", c_void_p),
+                ("scalar_stride", c_int64 * 3), ("vector_stride", c_int64 * 4), ("dtype", c_int32), ("pad", c_int32)]
+
+
 EXPORTED = ("lbm355_sweep", "lbm355_table_elements", "lbm355_noslip_links", "lbm355_reduce_conserved",
             "lbm355_count_nonfinite",
-            "lbm355_set_equilibrium", "lbm355_get_macroscopic", "lbm355_stream_copy", "lbm355_desc_size",
+            "lbm355_set_equilibrium", "lbm355_get_macroscopic", "lbm355_get_fields", "lbm355_stream_copy", "lbm355_desc_size",
             "lbm355_last_error", "lbm355_version", "lbm355_batch_create", "lbm355_batch_sweep",
             "lbm355_batch_info", "lbm355_batch_destroy", "lbm355_batch_sweep_static", "lbm355_closure_params_size",
             "lbm355_closure_master_size", "lbm355_closure_features", "lbm355_closure_forward",
@@ -97,6 +102,9 @@ def load(path=None):
     lib.lbm355_get_macroscopic.argtypes = [ctypes.POINTER(SweepDesc), c_void_p, c_void_p, c_void_p, c_int32,
                                            c_void_p]
     lib.lbm355_get_macroscopic.restype = c_int32
+    lib.lbm355_get_fields.argtypes = [ctypes.POINTER(SweepDesc), c_void_p, ctypes.POINTER(MacroscopicOut), c_int32,
+                                      c_void_p]
+    lib.lbm355_get_fields.restype = c_int32
     lib.lbm355_stream_copy.argtypes = [c_void_p, c_void_p, c_int64, c_int32, c_void_p]
     lib.lbm355_stream_copy.restype = c_int32
     lib.lbm355_plane_copy.argtypes = [c_int32, c_int32, c_void_p, c_void_p, c_int64, c_int64, c_int32, c_int32,

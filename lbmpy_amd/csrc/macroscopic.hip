@@ -119,22 +119,31 @@ __global__ void set_equilibrium_kernel(TS* pdf, const double* rho_in, const doub
   }
 }
 
+// What a getter reads, and where it writes: field element (x, y, z, c) of the interior at x stride[0] + y stride[1] +
+// z stride[2] + c stride[3] elements (float or double) from its pointer; a null pointer leaves the field out.
+struct GetArgs {
+  int nx, ny, nz, g;
+  int64_t sy, sz, sq;
+  int face[3];
+  int flags;
+  double force[3];
+  CellDivider row, plane;
+  lbm355_macroscopic_out out;
+};
+
+// density and velocity of one cell from the populations the last kernel wrote
 template <class S, int PAT, class TS>
-__global__ void get_macroscopic_kernel(const TS* pdf, double* rho_out, double* u_out, int nx, int ny, int nz, int g,
-                                       int64_t sy, int64_t sz, int64_t sq, int64_t osy, int64_t osz, int64_t osc,
-                                       int fx_mode, int fy_mode, int fz_mode, int flags, double fx, double fy,
-                                       double fz) {
+__device__ __forceinline__ void cell_macroscopic(const TS* pdf, const GetArgs& a, int x, int y, int z, double& rho,
+                                                 double (&u)[3]) {
   constexpr int Q = S::Q, D = S::D;
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= nx) return;
-  const int y = blockIdx.y, z = blockIdx.z;
-  const AxisNb ax = axis_neighbours(x, nx, g, fx_mode);
-  const AxisNb ay = axis_neighbours(y, ny, g, fy_mode);
+  const AxisNb ax = axis_neighbours(x, a.nx, a.g, a.face[0]);
+  const AxisNb ay = axis_neighbours(y, a.ny, a.g, a.face[1]);
   AxisNb az = {0, 0, false, false};
-  if (D == 3) az = axis_neighbours(z, nz, g, fz_mode);
-  const int64_t X[3] = {ax.lo, x + g, ax.hi};
-  const int64_t Y[3] = {ay.lo * sy, (y + g) * sy, ay.hi * sy};
-  const int64_t Z[3] = {D == 3 ? az.lo * sz : 0, D == 3 ? (z + g) * sz : 0, D == 3 ? az.hi * sz : 0};
+  if (D == 3) az = axis_neighbours(z, a.nz, a.g, a.face[2]);
+  const int64_t sy = a.sy, sz = a.sz, sq = a.sq;
+  const int64_t X[3] = {ax.lo, x + a.g, ax.hi};
+  const int64_t Y[3] = {ay.lo * sy, (y + a.g) * sy, ay.hi * sy};
+  const int64_t Z[3] = {D == 3 ? az.lo * sz : 0, D == 3 ? (z + a.g) * sz : 0, D == 3 ? az.hi * sz : 0};
   const int64_t center = X[1] + Y[1] + Z[1];
   double s = 0, j[3] = {0, 0, 0};
 #pragma unroll
@@ -154,18 +163,87 @@ __global__ void get_macroscopic_kernel(const TS* pdf, double* rho_out, double* u
     j[1] += cy * v;
     j[2] += cz * v;
   }
-  const double rho = (flags & LBM355_FLAG_ZERO_CENTERED) ? 1.0 + s : s;
-  const double ref = (flags & LBM355_FLAG_COMPRESSIBLE) ? rho : 1.0;
-  const double F[3] = {fx, fy, fz};
-  const int64_t o = (int64_t)(x + g) + (int64_t)(y + g) * osy + (D == 3 ? (int64_t)(z + g) * osz : 0);
-  if (rho_out) rho_out[o] = rho;
-  if (u_out) {
+  rho = (a.flags & LBM355_FLAG_ZERO_CENTERED) ? 1.0 + s : s;
+  const double ref = (a.flags & LBM355_FLAG_COMPRESSIBLE) ? rho : 1.0;
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-      double ud = j[d] / ref;
-      if (flags & LBM355_FLAG_FORCE) ud += 0.5 * F[d] / ref;
-      u_out[o + d * osc] = ud;
+  for (int d = 0; d < D; ++d) {
+    double ud = j[d] / ref;
+    if (a.flags & LBM355_FLAG_FORCE) ud += 0.5 * a.force[d] / ref;
+    u[d] = ud;
+  }
+}
+
+__device__ __forceinline__ void put(void* p, int64_t at, double v, bool f32) {
+  if (f32)
+    ((float*)p)[at] = (float)v;
+  else
+    ((double*)p)[at] = v;
+}
+
+// Outputs with x fastest: one thread per cell, numbered consecutively.  Bound by memory: Q s bytes read and the fields
+// written, nothing in between (D3Q19 FP32 192x160x144 into FP32 fields: staging in FP64 and converting took 79 us for
+// this kernel and 60 for the conversions).
+template <class S, int PAT, class TS>
+__global__ void __launch_bounds__(256) get_macroscopic_kernel(const TS* pdf, GetArgs a) {
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t r = a.row.quotient(t), p = a.plane.quotient(r);
+  const int x = (int)(t - r * a.row.d), y = (int)(r - p * a.plane.d), z = (int)p;
+  if (t >= a.row.d * a.plane.d * (uint32_t)a.nz) return;
+  double rho, u[3];
+  cell_macroscopic<S, PAT, TS>(pdf, a, x, y, z, rho, u);
+  const lbm355_macroscopic_out& o = a.out;
+  const bool f32 = o.dtype == LBM355_F32;
+  const int64_t so = x * o.scalar_stride[0] + y * o.scalar_stride[1] + z * o.scalar_stride[2];
+  const int64_t vo = x * o.vector_stride[0] + y * o.vector_stride[1] + z * o.vector_stride[2];
+  if (o.density) put(o.density, so, rho, f32);
+  if (o.density_deviation) put(o.density_deviation, so, rho - 1.0, f32);
+  if (o.velocity) {
+#pragma unroll
+    for (int d = 0; d < S::D; ++d) put(o.velocity, vo + d * o.vector_stride[3], u[d], f32);
+  }
+}
+
+// Outputs with another order (numpy's [x][y][z][component], z or the component fastest): the populations are read along
+// x, 64 cells a wavefront, and the fields written along the last axis, so a block takes 64 x TURN cells of the plane of
+// x and the last axis and turns them in LDS.  The rows of 65 doubles put neither side's lanes on the same banks.
+constexpr int TURN = 16;
+template <class S, int PAT, class TS>
+__global__ void __launch_bounds__(256) get_turned_kernel(const TS* pdf, GetArgs a) {
+  constexpr int D = S::D;
+  __shared__ double field[1 + D][TURN][65];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int x0 = blockIdx.x * 64, l0 = blockIdx.y * TURN, n_last = D == 3 ? a.nz : a.ny;
+  const int nl = n_last - l0 < TURN ? n_last - l0 : TURN, nx = a.nx - x0 < 64 ? a.nx - x0 : 64;
+  const int y0 = D == 3 ? blockIdx.z : 0;
+  for (int l = wv; l < nl; l += 4) {
+    if (lane < nx) {
+      double rho, u[3];
+      cell_macroscopic<S, PAT, TS>(pdf, a, x0 + lane, D == 3 ? y0 : l0 + l, D == 3 ? l0 + l : 0, rho, u);
+      field[0][l][lane] = rho;
+#pragma unroll
+      for (int d = 0; d < D; ++d) field[1 + d][l][lane] = u[d];
     }
+  }
+  __syncthreads();
+  const lbm355_macroscopic_out& o = a.out;
+  const bool f32 = o.dtype == LBM355_F32;
+  constexpr int LAST = D - 1;
+  const int64_t so = x0 * o.scalar_stride[0] + l0 * o.scalar_stride[LAST] + (D == 3 ? y0 * o.scalar_stride[1] : 0);
+  const int64_t vo = x0 * o.vector_stride[0] + l0 * o.vector_stride[LAST] + (D == 3 ? y0 * o.vector_stride[1] : 0);
+  for (int e = threadIdx.x; e < nx * TURN; e += 256) {
+    const int l = e % TURN, x = e / TURN;
+    if (l >= nl) continue;
+    const double rho = field[0][l][x];
+    const int64_t at = so + x * o.scalar_stride[0] + l * o.scalar_stride[LAST];
+    if (o.density) put(o.density, at, rho, f32);
+    if (o.density_deviation) put(o.density_deviation, at, rho - 1.0, f32);
+  }
+  if (!o.velocity) return;
+  for (int e = threadIdx.x; e < nx * TURN * D; e += 256) {
+    const int d = e % D, l = (e / D) % TURN, x = e / (D * TURN);
+    if (l >= nl) continue;
+    put(o.velocity, vo + x * o.vector_stride[0] + l * o.vector_stride[LAST] + d * o.vector_stride[3], field[1 + d][l][x],
+        f32);
   }
 }
 
@@ -259,27 +337,31 @@ int set_eq_launch(const lbm355_sweep_desc* d, void* pdf, const double* rho, cons
   return hipGetLastError() == hipSuccess ? 0 : fail2(LBM355_ERR_LAUNCH, "setter launch failed");
 }
 
-template <class S, class TS>
-int get_launch(const lbm355_sweep_desc* d, const void* pdf, double* rho, double* u, int last_pattern,
-               hipStream_t s) {
-  const int bx = d->nx >= 256 ? 256 : ((d->nx + 63) / 64) * 64;
-  dim3 block(bx), grid((d->nx + bx - 1) / bx, d->ny, d->nz);
-  decltype(&get_macroscopic_kernel<S, LBM355_PULL, TS>) k = nullptr;
+template <class S, class TS, bool TURNED>
+int get_launch(const GetArgs& a, const void* pdf, int last_pattern, hipStream_t s) {
+  const int64_t cells = (int64_t)a.nx * a.ny * a.nz;
+  dim3 grid((unsigned)((cells + 255) / 256)), block(256);
+  if (TURNED) grid = dim3((a.nx + 63) / 64, ((S::D == 3 ? a.nz : a.ny) + TURN - 1) / TURN, S::D == 3 ? a.ny : 1);
+#define LBM_GET(P)                                                                                       \
+  case P:                                                                                                \
+    if constexpr (TURNED)                                                                                \
+      hipLaunchKernelGGL((get_turned_kernel<S, P, TS>), grid, block, 0, s, (const TS*)pdf, a);           \
+    else                                                                                                 \
+      hipLaunchKernelGGL((get_macroscopic_kernel<S, P, TS>), grid, block, 0, s, (const TS*)pdf, a);      \
+    break;
   switch (last_pattern) {
-    case LBM355_PULL: k = get_macroscopic_kernel<S, LBM355_PULL, TS>; break;
-    case LBM355_AA_EVEN: k = get_macroscopic_kernel<S, LBM355_AA_EVEN, TS>; break;
-    case LBM355_AA_ODD: k = get_macroscopic_kernel<S, LBM355_AA_ODD, TS>; break;
-    case LBM355_ESOTWIST_EVEN: k = get_macroscopic_kernel<S, LBM355_ESOTWIST_EVEN, TS>; break;
-    case LBM355_ESOTWIST_ODD: k = get_macroscopic_kernel<S, LBM355_ESOTWIST_ODD, TS>; break;
-    case LBM355_ESOPULL_EVEN: k = get_macroscopic_kernel<S, LBM355_ESOPULL_EVEN, TS>; break;
-    case LBM355_ESOPULL_ODD: k = get_macroscopic_kernel<S, LBM355_ESOPULL_ODD, TS>; break;
-    case LBM355_ESOPUSH_EVEN: k = get_macroscopic_kernel<S, LBM355_ESOPUSH_EVEN, TS>; break;
-    case LBM355_ESOPUSH_ODD: k = get_macroscopic_kernel<S, LBM355_ESOPUSH_ODD, TS>; break;
-    default: k = get_macroscopic_kernel<S, LBM355_PUSH, TS>; break;
+    LBM_GET(LBM355_PULL)
+    LBM_GET(LBM355_AA_EVEN)
+    LBM_GET(LBM355_AA_ODD)
+    LBM_GET(LBM355_ESOTWIST_EVEN)
+    LBM_GET(LBM355_ESOTWIST_ODD)
+    LBM_GET(LBM355_ESOPULL_EVEN)
+    LBM_GET(LBM355_ESOPULL_ODD)
+    LBM_GET(LBM355_ESOPUSH_EVEN)
+    LBM_GET(LBM355_ESOPUSH_ODD)
+    LBM_GET(LBM355_PUSH)
   }
-  hipLaunchKernelGGL(k, grid, block, 0, s, (const TS*)pdf, rho, u, d->nx, d->ny, d->nz, d->ghost_layers, d->stride_y,
-                     d->stride_z, d->stride_q, d->out_stride_y, d->out_stride_z, d->out_stride_c, d->face[0],
-                     d->face[1], d->face[2], d->flags, d->force[0], d->force[1], d->force[2]);
+#undef LBM_GET
   return hipGetLastError() == hipSuccess ? 0 : fail2(LBM355_ERR_LAUNCH, "getter launch failed");
 }
 
@@ -291,11 +373,34 @@ int set_eq_dtype(const lbm355_sweep_desc* d, void* pdf, const double* rho, const
   return set_eq_launch<S, FAM, _Float16>(d, pdf, rho, u, tab, prev, s);
 }
 
+template <class S, class TS>
+int get_order(const GetArgs& a, const void* pdf, int last, hipStream_t s) {
+  const bool x_first = (!(a.out.density || a.out.density_deviation) || a.out.scalar_stride[0] == 1) &&
+                       (!a.out.velocity || a.out.vector_stride[0] == 1);
+  return x_first ? get_launch<S, TS, false>(a, pdf, last, s) : get_launch<S, TS, true>(a, pdf, last, s);
+}
+
 template <class S>
-int get_dtype(const lbm355_sweep_desc* d, const void* pdf, double* rho, double* u, int last, hipStream_t s) {
-  if (d->store_dtype == LBM355_F64) return get_launch<S, double>(d, pdf, rho, u, last, s);
-  if (d->store_dtype == LBM355_F32) return get_launch<S, float>(d, pdf, rho, u, last, s);
-  return get_launch<S, _Float16>(d, pdf, rho, u, last, s);
+int get_dtype(const lbm355_sweep_desc* d, const void* pdf, const lbm355_macroscopic_out& out, int last, hipStream_t s) {
+  GetArgs a;
+  a.nx = d->nx;
+  a.ny = d->ny;
+  a.nz = d->nz;
+  a.g = d->ghost_layers;
+  a.sy = d->stride_y;
+  a.sz = d->stride_z;
+  a.sq = d->stride_q;
+  for (int k = 0; k < 3; ++k) {
+    a.face[k] = d->face[k];
+    a.force[k] = d->force[k];
+  }
+  a.flags = d->flags;
+  a.row = CellDivider::of((uint32_t)d->nx);
+  a.plane = CellDivider::of((uint32_t)d->ny);
+  a.out = out;
+  if (d->store_dtype == LBM355_F64) return get_order<S, double>(a, pdf, last, s);
+  if (d->store_dtype == LBM355_F32) return get_order<S, float>(a, pdf, last, s);
+  return get_order<S, _Float16>(a, pdf, last, s);
 }
 
 template <class S, int FAM>
@@ -350,19 +455,38 @@ int lbm355_set_equilibrium(const lbm355_sweep_desc* d, void* pdf, const double* 
   return fail2(LBM355_ERR_UNSUPPORTED, "no setter for this stencil/family");
 }
 
-int lbm355_get_macroscopic(const lbm355_sweep_desc* d, const void* pdf, double* density, double* velocity,
-                           int32_t last_pattern, void* stream) {
-  if (!d || !pdf) return fail2(LBM355_ERR_ARG, "NULL argument");
+int lbm355_get_fields(const lbm355_sweep_desc* d, const void* pdf, const lbm355_macroscopic_out* out,
+                      int32_t last_pattern, void* stream) {
+  if (!d || !pdf || !out) return fail2(LBM355_ERR_ARG, "NULL argument");
   if (d->store_dtype < 0 || d->store_dtype > 2) return fail2(LBM355_ERR_ARG, "bad dtype");
+  if (out->dtype != LBM355_F64 && out->dtype != LBM355_F32) return fail2(LBM355_ERR_ARG, "output fields are F64 or F32");
   if (last_pattern < LBM355_PULL || last_pattern > LBM355_PUSH) return fail2(LBM355_ERR_ARG, "bad pattern");
+  if (d->nx <= 0 || d->ny <= 0 || d->nz <= 0 || d->ny > 65535 || d->nz > 65535 ||
+      (int64_t)d->nx * d->ny * d->nz >= (int64_t(1) << 31))
+    return fail2(LBM355_ERR_ARG, "bad interior size");
   if (table_pattern(last_pattern))
     for (int a = 0; a < (d->stencil == LBM355_D2Q9 ? 2 : 3); ++a)
       if (d->face[a] == LBM355_FACE_NOSLIP) return fail2(LBM355_ERR_ARG, "Eso patterns have no fused NoSlip faces");
   hipStream_t s = (hipStream_t)stream;
-  if (d->stencil == LBM355_D2Q9) return get_dtype<D2Q9>(d, pdf, density, velocity, last_pattern, s);
-  if (d->stencil == LBM355_D3Q19) return get_dtype<D3Q19>(d, pdf, density, velocity, last_pattern, s);
-  if (d->stencil == LBM355_D3Q27) return get_dtype<D3Q27>(d, pdf, density, velocity, last_pattern, s);
+  if (d->stencil == LBM355_D2Q9) return get_dtype<D2Q9>(d, pdf, *out, last_pattern, s);
+  if (d->stencil == LBM355_D3Q19) return get_dtype<D3Q19>(d, pdf, *out, last_pattern, s);
+  if (d->stencil == LBM355_D3Q27) return get_dtype<D3Q27>(d, pdf, *out, last_pattern, s);
   return fail2(LBM355_ERR_ARG, "unknown stencil");
+}
+
+int lbm355_get_macroscopic(const lbm355_sweep_desc* d, const void* pdf, double* density, double* velocity,
+                           int32_t last_pattern, void* stream) {
+  if (!d) return fail2(LBM355_ERR_ARG, "NULL argument");
+  const int64_t first = d->ghost_layers * (1 + d->out_stride_y + (d->stencil == LBM355_D2Q9 ? 0 : d->out_stride_z));
+  lbm355_macroscopic_out out = {};
+  out.density = density ? density + first : nullptr;
+  out.velocity = velocity ? velocity + first : nullptr;
+  out.dtype = LBM355_F64;
+  out.scalar_stride[0] = out.vector_stride[0] = 1;
+  out.scalar_stride[1] = out.vector_stride[1] = d->out_stride_y;
+  out.scalar_stride[2] = out.vector_stride[2] = d->out_stride_z;
+  out.vector_stride[3] = d->out_stride_c;
+  return lbm355_get_fields(d, pdf, &out, last_pattern, stream);
 }
 
 int lbm355_get_strain_rate(const lbm355_sweep_desc* d, const void* pdf, const double* table_f64, double* strain_rate,

@@ -253,14 +253,17 @@ __global__ void zero4_kernel(double* out) {
   if (threadIdx.x < 4) out[threadIdx.x] = 0.0;
 }
 
+// Each thread sums many cells before the block's one atomic per sum: the 4 sums are one cache line, and atomics of all
+// blocks on it take their turns (one cell per thread: 92160 atomics and 291 us at D3Q19 FP32 192x160x144).
+constexpr unsigned REDUCE_BLOCKS = 512;
 template <class S, class TS>
-__global__ void __launch_bounds__(256) reduce_kernel(const TS* pdf, int nx, int ny, int nz, int g, int64_t sy,
-                                                     int64_t sz, int64_t sq, int zc, double* out) {
+__global__ void __launch_bounds__(256) reduce_kernel(const TS* pdf, CellDivider row, CellDivider plane, uint32_t cells,
+                                                     int g, int64_t sy, int64_t sz, int64_t sq, int zc, double* out) {
   constexpr int Q = S::Q;
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
-  const int y = blockIdx.y, z = blockIdx.z;
   double r = 0, jx = 0, jy = 0, jz = 0;
-  if (x < nx) {
+  for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < cells; t += gridDim.x * blockDim.x) {
+    const uint32_t l = row.quotient(t), p = plane.quotient(l);
+    const int x = (int)(t - l * row.d), y = (int)(l - p * plane.d), z = (int)p;
     const int64_t c = (x + g) + (y + g) * sy + (S::D == 3 ? (z + g) * sz : 0);
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
@@ -300,13 +303,15 @@ __global__ void zero1_kernel(unsigned long long* out) {
 }
 
 template <class S, class TS>
-__global__ void __launch_bounds__(256) nonfinite_kernel(const TS* pdf, int nx, int g, int64_t sy, int64_t sz,
-                                                        int64_t sq, unsigned long long* out) {
+__global__ void __launch_bounds__(256) nonfinite_kernel(const TS* pdf, CellDivider row, CellDivider plane, uint32_t cells,
+                                                        int g, int64_t sy, int64_t sz, int64_t sq,
+                                                        unsigned long long* out) {
   constexpr int Q = S::Q;
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
-  const int y = blockIdx.y, z = blockIdx.z;
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
   unsigned n = 0;
-  if (x < nx) {
+  if (t < cells) {
+    const uint32_t l = row.quotient(t), p = plane.quotient(l);
+    const int x = (int)(t - l * row.d), y = (int)(l - p * plane.d), z = (int)p;
     const int64_t c = (x + g) + (y + g) * sy + (S::D == 3 ? (z + g) * sz : 0);
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
@@ -345,18 +350,6 @@ namespace {
 
 template <class TC>
 using KernelFn = void (*)(SweepArgs<TC>);
-
-struct Launch {
-  dim3 grid, block;
-};
-
-Launch geometry(int nx, int ny, int nz) {
-  int bx = (nx >= 256 ? 256 : ((nx + 63) / 64) * 64);
-  Launch l;
-  l.block = dim3(bx, 1, 1);
-  l.grid = dim3((nx + bx - 1) / bx, ny, nz);
-  return l;
-}
 
 size_t elem_size(int dtype) { return dtype == LBM355_F64 ? 8 : (dtype == LBM355_F32 ? 4 : 2); }
 
@@ -563,11 +556,18 @@ int launch_bc_dtype(const lbm355_boundary_desc* d, void* pdf, const int32_t* lin
   return launch_bc<S, _Float16>(d, pdf, links, n, vel, b, s);
 }
 
+bool cells_below_2_31(const lbm355_sweep_desc* d) {
+  return d->nx > 0 && d->ny > 0 && d->nz > 0 && (int64_t)d->nx * d->ny < (int64_t(1) << 31) &&
+         (int64_t)d->nx * d->ny * d->nz < (int64_t(1) << 31);
+}
+
 template <class S, class TS>
 int launch_reduce(const lbm355_sweep_desc* d, const void* pdf, double* out, hipStream_t s) {
   hipLaunchKernelGGL(zero4_kernel, dim3(1), dim3(64), 0, s, out);
-  Launch l = geometry(d->nx, d->ny, d->nz);
-  hipLaunchKernelGGL((reduce_kernel<S, TS>), l.grid, l.block, 0, s, (const TS*)pdf, d->nx, d->ny, d->nz,
+  const uint32_t cells = (uint32_t)((int64_t)d->nx * d->ny * d->nz);
+  const unsigned blocks = (cells + 255) / 256;
+  hipLaunchKernelGGL((reduce_kernel<S, TS>), dim3(blocks < REDUCE_BLOCKS ? blocks : REDUCE_BLOCKS), dim3(256), 0, s,
+                     (const TS*)pdf, CellDivider::of((uint32_t)d->nx), CellDivider::of((uint32_t)d->ny), cells,
                      d->ghost_layers, d->stride_y, d->stride_z, d->stride_q,
                      (d->flags & LBM355_FLAG_ZERO_CENTERED) ? 1 : 0, out);
   hipError_t e = hipGetLastError();
@@ -578,8 +578,9 @@ int launch_reduce(const lbm355_sweep_desc* d, const void* pdf, double* out, hipS
 template <class S, class TS>
 int launch_nonfinite(const lbm355_sweep_desc* d, const void* pdf, unsigned long long* out, hipStream_t s) {
   hipLaunchKernelGGL(zero1_kernel, dim3(1), dim3(64), 0, s, out);
-  Launch l = geometry(d->nx, d->ny, d->nz);
-  hipLaunchKernelGGL((nonfinite_kernel<S, TS>), l.grid, l.block, 0, s, (const TS*)pdf, d->nx, d->ghost_layers,
+  const uint32_t cells = (uint32_t)((int64_t)d->nx * d->ny * d->nz);
+  hipLaunchKernelGGL((nonfinite_kernel<S, TS>), dim3((cells + 255) / 256), dim3(256), 0, s, (const TS*)pdf,
+                     CellDivider::of((uint32_t)d->nx), CellDivider::of((uint32_t)d->ny), cells, d->ghost_layers,
                      d->stride_y, d->stride_z, d->stride_q, out);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(LBM355_ERR_LAUNCH, std::string("launch failed: ") + hipGetErrorString(e));
@@ -763,6 +764,7 @@ int lbm355_boundary_links(const lbm355_boundary_desc* d, void* pdf, const int32_
 
 int lbm355_reduce_conserved(const lbm355_sweep_desc* d, const void* pdf, double* out, void* stream) {
   if (!d || !pdf || !out) return fail(LBM355_ERR_ARG, "NULL argument");
+  if (!cells_below_2_31(d)) return fail(LBM355_ERR_ARG, "bad interior size");
   hipStream_t s = (hipStream_t)stream;
   if (d->stencil == LBM355_D2Q9) return reduce_dtype<D2Q9>(d, pdf, out, s);
   if (d->stencil == LBM355_D3Q19) return reduce_dtype<D3Q19>(d, pdf, out, s);
@@ -772,7 +774,7 @@ int lbm355_reduce_conserved(const lbm355_sweep_desc* d, const void* pdf, double*
 
 int lbm355_count_nonfinite(const lbm355_sweep_desc* d, const void* pdf, uint64_t* out, void* stream) {
   if (!d || !pdf || !out) return fail(LBM355_ERR_ARG, "NULL argument");
-  if (d->nx <= 0 || d->ny <= 0 || d->nz <= 0) return fail(LBM355_ERR_ARG, "bad interior size");
+  if (!cells_below_2_31(d)) return fail(LBM355_ERR_ARG, "bad interior size");
   hipStream_t s = (hipStream_t)stream;
   unsigned long long* o = reinterpret_cast<unsigned long long*>(out);
   if (d->stencil == LBM355_D2Q9) return nonfinite_dtype<D2Q9>(d, pdf, o, s);

@@ -93,7 +93,7 @@ class _Context:
             f = self._staging[key] = f.permute(*reversed(range(1, self.D + 1)), 0)
         return f
 
-    def descriptor(self, pdfs, rho, u):
+    def descriptor(self, pdfs, rho=None, u=None):
         m = self.method
         D, g = self.D, self.g
         d = nat.SweepDesc()
@@ -112,9 +112,10 @@ class _Context:
         d.stride_y = pdfs.stride(1)
         d.stride_z = pdfs.stride(2) if D == 3 else 0
         d.stride_q = pdfs.stride(D)
-        d.out_stride_y = rho.stride(1)
-        d.out_stride_z = rho.stride(2) if D == 3 else 0
-        d.out_stride_c = u.stride(D)
+        if rho is not None:
+            d.out_stride_y = rho.stride(1)
+            d.out_stride_z = rho.stride(2) if D == 3 else 0
+            d.out_stride_c = u.stride(D)
         flags = 0
         if m.zero_centered_pdfs:
             flags |= nat.FLAG_ZERO_CENTERED
@@ -164,8 +165,43 @@ def _set(ctx, pdfs, density, velocity, code):
                                          nat.current_stream_handle()))
 
 
+def _get_in_place(ctx, pdfs, density, velocity, code, density_deviation):
+    """The getter straight into the output tensors; False where they do not admit it (the kernel takes FP64 and FP32
+    fields of any order, shaped like the PDFs)."""
+    D, g = ctx.D, ctx.g
+    spatial = tuple(pdfs.shape[:-1])
+    scalars = [t for t in (density, density_deviation) if t is not None]
+    fields = scalars + ([velocity] if velocity is not None else [])
+    if not all(isinstance(t, torch.Tensor) and t.device == pdfs.device and not t.requires_grad for t in fields) or \
+            len({t.dtype for t in fields}) != 1 or fields[0].dtype not in (torch.float64, torch.float32) or \
+            any(tuple(t.shape) != spatial for t in scalars) or len({t.stride() for t in scalars}) > 1 or \
+            (velocity is not None and tuple(velocity.shape) != spatial + (D,)) or \
+            any(n > 1 and s == 0 for t in fields for n, s in zip(t.shape, t.stride())):
+        return False
+    o = nat.MacroscopicOut()
+    o.dtype = nat.F64 if fields[0].dtype == torch.float64 else nat.F32
+    if scalars:
+        for a in range(D):
+            o.scalar_stride[a] = scalars[0].stride(a)
+    if velocity is not None:
+        for a in range(D):
+            o.vector_stride[a] = velocity.stride(a)
+        o.vector_stride[3] = velocity.stride(D)
+    inner = tuple(slice(g, s - g) for s in spatial)
+    for name, t in (("density", density), ("density_deviation", density_deviation), ("velocity", velocity)):
+        if t is not None:
+            setattr(o, name, t[inner].data_ptr())
+    d = ctx.descriptor(pdfs)
+    nat.check(nat.load().lbm355_get_fields(ctypes.byref(d), ctypes.c_void_p(pdfs.data_ptr()), ctypes.byref(o), code,
+                                           nat.current_stream_handle()))
+    return True
+
+
 def _get(ctx, pdfs, density, velocity, code, density_deviation=None):
     ctx.check_pdfs(pdfs)
+    if (density is not None or density_deviation is not None or velocity is not None) and \
+            _get_in_place(ctx, pdfs, density, velocity, code, density_deviation):
+        return
     rho, u = ctx.fields(pdfs)
     d = ctx.descriptor(pdfs, rho, u)
     lib = nat.load()

@@ -394,7 +394,7 @@ class SweepKernel:
         self._check_tensor(pdf)
         binds = {s: float(bindings.get(s, 1.0)) for s in self.free_symbols}
         d = self.descriptor(pdf, binds)
-        out = torch.zeros(4, dtype=torch.float64, device=pdf.device)
+        out = torch.empty(4, dtype=torch.float64, device=pdf.device)
         lib = nat.load()
         nat.check(lib.lbm355_reduce_conserved(ctypes.byref(d), ctypes.c_void_p(pdf.data_ptr()),
                                               ctypes.c_void_p(out.data_ptr()), nat.current_stream_handle()))
@@ -406,7 +406,7 @@ class SweepKernel:
         self._check_tensor(pdf)
         binds = {s: float(bindings.get(s, 1.0)) for s in self.free_symbols}
         d = self.descriptor(pdf, binds)
-        out = torch.zeros(1, dtype=torch.int64, device=pdf.device)
+        out = torch.empty(1, dtype=torch.int64, device=pdf.device)
         lib = nat.load()
         nat.check(lib.lbm355_count_nonfinite(ctypes.byref(d), ctypes.c_void_p(pdf.data_ptr()),
                                              ctypes.c_void_p(out.data_ptr()), nat.current_stream_handle()))
