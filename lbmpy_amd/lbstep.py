@@ -109,8 +109,11 @@ class LatticeBoltzmannStep:
         self._src = create_pdf_array(domain_size, q, 1, dt)
         self._tmp = create_pdf_array(domain_size, q, 1, dt) if self._two_arrays else None
         # macroscopic fields: host numpy (interior) + FP64 device staging with the PDF ghost layout
-        self._rho_host = np.ones(domain_size)
-        self._u_host = np.zeros(domain_size + (dim,))
+        # (pinned memory, which the getter's kernel writes directly)
+        self._rho_pinned = torch.ones(domain_size, dtype=torch.float64, pin_memory=True)
+        self._u_pinned = torch.zeros(domain_size + (dim,), dtype=torch.float64, pin_memory=True)
+        self._rho_host = self._rho_pinned.numpy()
+        self._u_host = self._u_pinned.numpy()
         self._rho_dev = torch.zeros([n + 2 for n in domain_size][::-1], dtype=torch.float64, device="cuda")
         self._u_dev = torch.zeros([dim] + [n + 2 for n in domain_size][::-1], dtype=torch.float64, device="cuda")
         self._boundary_handling = LatticeBoltzmannBoundaryHandling.for_domain(self.method, domain_size,
@@ -208,9 +211,9 @@ class LatticeBoltzmannStep:
         """Equilibrium from the host density/velocity fields (lbstep.py:268-269), on the GPU."""
         D = self.dim
         inner = (slice(1, -1),) * D
-        self._rho_dev[inner] = torch.from_numpy(np.ascontiguousarray(self._rho_host.T)).cuda()
-        for a in range(D):
-            self._u_dev[a][inner] = torch.from_numpy(np.ascontiguousarray(self._u_host[..., a].T)).cuda()
+        back = tuple(range(D - 1, -1, -1))
+        self._rho_dev[inner] = self._rho_pinned.cuda(non_blocking=True).permute(*back)
+        self._u_dev[(slice(None),) + inner] = self._u_pinned.cuda(non_blocking=True).permute(D, *back)
         d = self._descriptor()
         tab, _ = method_table(self.method, self.kernel_params, np.float64,
                               corrections=self._kernels[0].corrections)
@@ -254,16 +257,22 @@ class LatticeBoltzmannStep:
             last = self._codes[0]
         else:
             last = self._codes[0] if self._aa_next_odd else self._codes[1]
-        lib = nat.load()
-        nat.check(lib.lbm355_get_macroscopic(ctypes.byref(d), ctypes.c_void_p(self._src.data_ptr()),
-                                             ctypes.c_void_p(self._rho_dev.data_ptr()),
-                                             ctypes.c_void_p(self._u_dev.data_ptr()), last,
-                                             nat.current_stream_handle()))
+        # The kernel writes the host fields themselves, in numpy's order, over the bus: one launch and one wait.  On
+        # MI355X 96^3 (28 MB) takes 0.56 ms, 50 GB/s, where pageable copies of x-fastest fields and numpy's transposition
+        # took 12 ms; 40x80 takes 18 us.  (Staging on the device and one copy is 16 us slower there, and 7% faster at best
+        # above 30 MB.)
+        out = nat.MacroscopicOut()
+        out.dtype = nat.F64
+        out.density = self._rho_pinned.data_ptr()
+        out.velocity = self._u_pinned.data_ptr()
         D = self.dim
-        inner = (slice(1, -1),) * D
-        self._rho_host[...] = self._rho_dev[inner].cpu().numpy().T
         for a in range(D):
-            self._u_host[..., a] = self._u_dev[a][inner].cpu().numpy().T
+            out.scalar_stride[a] = self._rho_pinned.stride(a)
+            out.vector_stride[a] = self._u_pinned.stride(a)
+        out.vector_stride[3] = self._u_pinned.stride(D)
+        nat.check(nat.load().lbm355_get_fields(ctypes.byref(d), ctypes.c_void_p(self._src.data_ptr()),
+                                               ctypes.byref(out), last, nat.current_stream_handle()))
+        torch.cuda.current_stream().synchronize()
 
     # ------------------------------------------------------------------ fixed two-step loop
     # lbmpy's run() and benchmark_run() go through a time loop of two fixed steps with the kernel arguments bound
