@@ -203,38 +203,30 @@ __device__ __forceinline__ void collide_cell(TC (&f)[S::Q], const SweepArgs<TC>&
 }
 
 // Loads and stores of element `off` (0 <= off < 2^31) of a population plane.  With 2-byte storage the byte offset
-// fits in 32 bits (a plane holds < 2^31 elements), so they are raw buffer accesses: the plane's base lives in a
-// buffer descriptor that scalar instructions build, one 32-bit vector offset serves every plane, and no population
-// needs 64-bit address arithmetic.  Wider storage uses ordinary pointers.  NT: non-temporal.
-constexpr int BUFFER_DWORD3 = 0x00020000;   // raw (untyped) buffer access on gfx9 family targets
+// fits in 32 bits (a plane holds < 2^31 elements): the accesses take the plane's base from scalar registers and one
+// 32-bit vector offset for every plane.  They are global accesses: the base in a buffer descriptor has to lie on a
+// dword, which every other plane of an odd number of elements does not, and near walls, where the lanes of a wavefront
+// differ in plane, each descriptor takes a pass of its own (D3Q27 cumulant 250x200x180 AA: 173 us with descriptors,
+// 170 without).  Wider storage uses ordinary pointers.  NT: non-temporal.
+template <class TS>
+__device__ __forceinline__ TS* plane_at(TS* plane, int off) {
+  using Byte = std::conditional_t<std::is_const<TS>::value, const char, char>;
+  if constexpr (sizeof(TS) == 2) return reinterpret_cast<TS*>(reinterpret_cast<Byte*>(plane) + (uint32_t)off * 2u);
+  return plane + off;
+}
 
 template <class TS, class TC, bool NT>
 __device__ __forceinline__ TC plane_load(const TS* plane, int off) {
-  if constexpr (sizeof(TS) == 2) {
-    const __amdgpu_buffer_rsrc_t r =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<TS*>(plane), (short)0, -1, BUFFER_DWORD3);
-    const unsigned short bits = __builtin_amdgcn_raw_buffer_load_b16(r, (int)((uint32_t)off * 2u), 0, NT ? 2 : 0);
-    TS v;
-    __builtin_memcpy(&v, &bits, 2);
-    return (TC)v;
-  } else {
-    return NT ? load_nt<TS, TC>(plane + off) : load_as<TS, TC>(plane + off);
-  }
+  const TS* p = plane_at(plane, off);
+  return NT ? load_nt<TS, TC>(p) : load_as<TS, TC>(p);
 }
 template <class TS, class TC, bool NT>
 __device__ __forceinline__ void plane_store(TS* plane, int off, TC value) {
-  if constexpr (sizeof(TS) == 2) {
-    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(plane, (short)0, -1, BUFFER_DWORD3);
-    const TS v = (TS)value;
-    unsigned short bits;
-    __builtin_memcpy(&bits, &v, 2);
-    __builtin_amdgcn_raw_buffer_store_b16(bits, r, (int)((uint32_t)off * 2u), 0, NT ? 2 : 0);
-  } else {
-    if (NT)
-      store_nt<TS, TC>(plane + off, value);
-    else
-      store_as<TS, TC>(plane + off, value);
-  }
+  TS* p = plane_at(plane, off);
+  if (NT)
+    store_nt<TS, TC>(p, value);
+  else
+    store_as<TS, TC>(p, value);
 }
 
 // One cell of the sweep with direct (non-LDS) addressing: load with streaming, collide, store.
@@ -391,7 +383,7 @@ inline bool starts_lines(const lbm355_sweep_desc* d, const void* src, const void
 //   pull 128x128x96 43.6 -> 33.0.  One run of blocks per XCD keeps a cell's neighbours in its L2 as well: D3Q19 SRT
 //   FP64 64x32x32 9.8 -> 7.4.  (The row kernel with regular accesses gave 61.2 at 128^3.)
 // - Above that, lines that start with a wavefront are best streamed past the caches, as they come: 256^3 593 (685 with
-//   regular accesses, 640 with runs of 16 blocks per XCD), FP16 250x200x180 252 -> 173.
+//   regular accesses, 640 with runs of 16 blocks per XCD), FP16 250x200x180 252 -> 170.
 // - Otherwise two wavefronts share most lines, and non-temporal accesses move those twice; regular ones, with
 //   neighbouring blocks on one XCD, do not: 256^3 with ghost layers 947 -> 709 (809 without the runs), 251x255x253
 //   793 -> 684, FP64 131x117x101 143 -> 121.
