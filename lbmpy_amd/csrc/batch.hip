@@ -64,7 +64,8 @@ __device__ __forceinline__ SweepArgs<TC> load_args(const CONST_AS SweepArgs<TC>*
   a.u_in = nullptr;
   a.nut_scale = TC(0);
   a.seed = 0;
-  a.order = XcdOrder::of(1);
+  a.order = XcdOrder::of(1, 1);
+  a.block = 0;
   return a;
 }
 

@@ -41,6 +41,7 @@ __device__ __forceinline__ void collide_moment(T (&f)[S::Q], const SweepArgs<T>&
   using L = MomentTab<Q>;
   const TablePtr<T> __restrict__ tab = table_ptr(a.tab);
 
+  warm_table<L::COEF, T>(tab);
   T s = 0, j[3] = {0, 0, 0};
 #pragma unroll
   for (int i = 0; i < Q; ++i) {

@@ -195,13 +195,13 @@ struct CellDivider {
 // `chunk` neighbouring block numbers share an XCD: within every group of 8 chunk blocks, the blocks of one XCD take
 // one run.  The blocks after the last whole group, and all of them with chunk <= 1, keep their numbers.
 struct XcdOrder {
-  uint32_t chunk;
+  uint32_t blocks, chunk;
   CellDivider group;
-  __host__ __device__ static XcdOrder of(uint32_t chunk) {
+  __host__ __device__ static XcdOrder of(uint32_t blocks, uint32_t chunk) {
     if (chunk < 1) chunk = 1;
-    return {chunk, CellDivider::of(8 * chunk)};
+    return {blocks, chunk, CellDivider::of(8 * chunk)};
   }
-  __host__ __device__ __forceinline__ uint32_t number(uint32_t block, uint32_t blocks) const {
+  __host__ __device__ __forceinline__ uint32_t number(uint32_t block) const {
     const uint32_t first = group.quotient(block) * group.d, k = block - first;
     return first + group.d > blocks ? block : first + (k & 7) * chunk + (k >> 3);
   }
@@ -234,6 +234,7 @@ struct SweepArgs {
   uint32_t seed;              // stochastic FP16 rounding: this launch's seed
   CellDivider row, plane;     // division by nx and by ny (thread_cell)
   XcdOrder order;             // of the blocks (thread_cell)
+  uint32_t block;             // threads per block: blockDim.x would be a load of its own, waited for before the first
 };
 
 // What a collision hands back to the cell beyond the populations: the Smagorinsky shear rate and Pi
@@ -252,6 +253,24 @@ using TablePtr = const __attribute__((address_space(4))) T*;
 template <class T>
 __device__ __forceinline__ TablePtr<T> table_ptr(const T* p) {
   return (TablePtr<T>)p;
+}
+
+// Brings the first N entries of a table into the scalar cache while the populations are on their way.  A wavefront reads
+// its table in many small batches, as many as scalar registers take, one after the other; each that misses waits for
+// the L2.  That is most of a small launch: with threads per block passed along instead of loaded,
+// D2Q9 SRT FP64 40x80 3.4 -> 3.0 us, D3Q19 SRT FP64 64x32x32 7.3 -> 6.4, 64^3 8.5 -> 6.9, TRT 96^3 AA 25.1 -> 22.7;
+// 256^3 is as fast with it as without.
+template <int N, class T>
+__device__ __forceinline__ void warm_table(TablePtr<T> tab) {
+  const TablePtr<uint32_t> words = (TablePtr<uint32_t>)tab;
+  constexpr int WORDS = N * sizeof(T) / 4, LINE = 16, AT_ONCE = 8;   // a few lines at once: the words take registers
+#pragma unroll
+  for (int first = 0; first < WORDS; first += LINE * AT_ONCE) {
+    uint32_t any = 0;
+#pragma unroll
+    for (int at = first; at < first + LINE * AT_ONCE && at < WORDS; at += LINE) any |= words[at];
+    asm volatile("" ::"s"(any));
+  }
 }
 
 // ---------------------------------------------------------------- addressing

@@ -460,6 +460,7 @@ int launch_sweep(const lbm355_sweep_desc* d, const void* src, void* dst, void* r
   if (!k) return fail(LBM355_ERR_UNSUPPORTED, "no kernel for this stencil/family/dtype combination");
   SweepArgs<TC> a = make_args<TC>(d, src, dst, rho, u);
   a.order = l.order;
+  a.block = l.block.x;
   hipLaunchKernelGGL((KernelFn<TC>)k, l.grid, l.block, launch_lds(d, l, walls, l.mode == ACCESS_ROWS ? lds : 0), s, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(LBM355_ERR_LAUNCH, std::string("launch failed: ") + hipGetErrorString(e));

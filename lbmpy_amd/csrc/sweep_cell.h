@@ -356,12 +356,12 @@ enum AccessMode { ACCESS_ROWS, ACCESS_WAVES, ACCESS_LINES, ACCESS_CACHED };
 template <int MODE, class TC>
 __device__ __forceinline__ bool thread_cell(const SweepArgs<TC>& a, int& x, int& y, int& z) {
   if constexpr (MODE == ACCESS_WAVES) {
-    x = blockIdx.x * blockDim.x + threadIdx.x;
+    x = blockIdx.x * a.block + threadIdx.x;
     y = blockIdx.y;
     z = blockIdx.z;
     return x < a.nx;
   }
-  const uint32_t t = a.order.number(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const uint32_t t = a.order.number(blockIdx.x) * a.block + threadIdx.x;
   const uint32_t r = a.row.quotient(t), p = a.plane.quotient(r);
   x = (int)(t - r * a.row.d);
   y = (int)(r - p * a.plane.d);
@@ -388,13 +388,13 @@ inline bool starts_lines(const lbm355_sweep_desc* d, const void* src, const void
 // - What fits the Infinity Cache (fits_cache) is found there by the next step, if it was written with regular stores:
 //   64^3 13.1 -> 10.0, 128^3 81.8 -> 56.7, 128^3 with ghost layers 145 -> 61, EsoTwist 100x90x80 28.2 -> 23.5, D3Q19 TRT
 //   pull 128x128x96 43.6 -> 33.0.  One run of blocks per XCD keeps a cell's neighbours in its L2 as well: D3Q19 SRT
-//   FP64 64x32x32 9.8 -> 7.4.  (The row kernel with regular accesses gave 61.2 at 128^3.)
+//   FP64 64x32x32 9.8 -> 6.4.  (The row kernel with regular accesses gave 61.2 at 128^3.)
 // - Above that, lines that start with a wavefront are best streamed past the caches, as they come: 256^3 593 (685 with
 //   regular accesses, 640 with runs of 16 blocks per XCD), FP16 250x200x180 252 -> 170.
 // - Otherwise two wavefronts share most lines, and non-temporal accesses move those twice; regular ones, with
 //   neighbouring blocks on one XCD, do not: 256^3 with ghost layers 947 -> 709 (809 without the runs), 251x255x253
-//   793 -> 684, FP64 131x117x101 143 -> 121.
-// Full wavefronts whatever nx is matter most for short rows: D3Q19 TRT 35x148x256 84 -> 31.
+//   793 -> 684, FP64 131x117x101 143 -> 117.
+// Full wavefronts whatever nx is matter most for short rows: D3Q19 TRT 35x148x256 84 -> 28.
 constexpr uint32_t SHARED_LINES_CHUNK = 16;
 constexpr int64_t SMALL_CELLS = 1 << 18;   // below: blocks of one wavefront, to spread over the 256 CUs
 
@@ -427,16 +427,16 @@ inline SweepLaunch sweep_launch(const lbm355_sweep_desc* d, const void* src, con
                                 bool waves_kernel, bool lines_kernel) {
   const bool fits = fits_cache(d, src == dst), half = population_bytes(d, src == dst) <= HALF_CACHE_BYTES;
   const bool lines = !fits && starts_lines(d, src, dst);
-  if (row_kernel && lines) return {ACCESS_ROWS, dim3(1, d->ny, d->nz), dim3(d->nx), XcdOrder::of(1), half};
+  if (row_kernel && lines) return {ACCESS_ROWS, dim3(1, d->ny, d->nz), dim3(d->nx), XcdOrder::of(1, 1), half};
   if (waves_kernel && lines && d->nx % 64 == 0) {
     const unsigned bx = d->nx < 256 ? d->nx : 256;
-    return {ACCESS_WAVES, dim3((d->nx + bx - 1) / bx, d->ny, d->nz), dim3(bx), XcdOrder::of(1), half};
+    return {ACCESS_WAVES, dim3((d->nx + bx - 1) / bx, d->ny, d->nz), dim3(bx), XcdOrder::of(1, 1), half};
   }
   const int64_t cells = (int64_t)d->nx * d->ny * d->nz;
   const unsigned bx = cells < SMALL_CELLS ? 64 : 256;
   const unsigned blocks = (unsigned)((cells + bx - 1) / bx);
-  if (lines_kernel && lines) return {ACCESS_LINES, dim3(blocks), dim3(bx), XcdOrder::of(1), half};
-  return {ACCESS_CACHED, dim3(blocks), dim3(bx), XcdOrder::of(fits ? blocks / 8 : SHARED_LINES_CHUNK), half};
+  if (lines_kernel && lines) return {ACCESS_LINES, dim3(blocks), dim3(bx), XcdOrder::of(blocks, 1), half};
+  return {ACCESS_CACHED, dim3(blocks), dim3(bx), XcdOrder::of(blocks, fits ? blocks / 8 : SHARED_LINES_CHUNK), half};
 }
 
 // Kernel arguments from a public descriptor (include/lbm355.h).
@@ -475,7 +475,8 @@ inline SweepArgs<TC> make_args(const lbm355_sweep_desc* d, const void* src, void
   a.seed = d->rounding_seed;
   a.row = CellDivider::of((uint32_t)d->nx);
   a.plane = CellDivider::of((uint32_t)d->ny);
-  a.order = XcdOrder::of(1);
+  a.order = XcdOrder::of(1, 1);
+  a.block = 0;
   return a;
 }
 

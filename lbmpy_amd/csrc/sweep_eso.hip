@@ -56,10 +56,12 @@ int lbm355_launch_sweep_eso(const lbm355_sweep_desc* d, const void* src, void* d
   if (d->compute_dtype == LBM355_F64) {
     SweepArgs<double> a = make_args<double>(d, src, dst, rho, u);
     a.order = l.order;
+    a.block = l.block.x;
     hipLaunchKernelGGL((void (*)(SweepArgs<double>))k, l.grid, l.block, shm, s, a);
   } else {
     SweepArgs<float> a = make_args<float>(d, src, dst, rho, u);
     a.order = l.order;
+    a.block = l.block.x;
     hipLaunchKernelGGL((void (*)(SweepArgs<float>))k, l.grid, l.block, shm, s, a);
   }
   hipError_t e = hipGetLastError();
