@@ -10,10 +10,10 @@
 // holds < 2^31 cells) and runs sweep_cell, the same per-cell function as the single-domain sweep
 // (sweep_cell.h): a member's cells get bit-identical results to a single-domain run of that member.
 //
-// Optional XCD-aware order: MI355X dispatches consecutive workgroups round-robin over its 8 XCDs
-// (each with its own L2).  With `xcd_order`, the workgroups of one XCD take one contiguous
-// stretch of the tile sequence, so the rows one tile's neighbour reads touch are fetched into the
-// same L2 that the neighbouring tiles are processed on.
+// XCD-aware order: MI355X dispatches consecutive workgroups round-robin over its 8 XCDs (each with its
+// own L2).  With `xcd_order`, and for an ensemble that fits the Infinity Cache, the workgroups of one XCD
+// take one contiguous stretch of the tile sequence, so the rows one tile's neighbour reads touch are
+// fetched into the same L2 that the neighbouring tiles are processed on (batch_access has the rest).
 #include <mutex>
 #include <string>
 #include <vector>
@@ -89,16 +89,14 @@ __host__ __device__ constexpr int batch_min_waves() {
   return 4;
 }
 
-template <class S, int FAM, int PAT, class TS, class TC>
+// NT: every member's cells start on lines (starts_lines).
+template <class S, int FAM, int PAT, bool NT, class TS, class TC>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(batch_min_waves<S, FAM, PAT, TS, TC>(), 8)))
 batch_kernel(const BatchEntry<TC>* __restrict__ members, const int32_t* __restrict__ tile_member, int64_t ntiles,
-             int swap, int xcd_order) {
-  const int waves_per_block = blockDim.x >> 6;
-  int b = blockIdx.x;
-  if (xcd_order && (gridDim.x & 7) == 0) b = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  const int64_t wave = (int64_t)b * waves_per_block + (threadIdx.x >> 6);
-  const int64_t nwaves = (int64_t)gridDim.x * waves_per_block;
+             int swap, int waves_per_block, XcdOrder order) {
+  const int64_t wave = (int64_t)order.number(blockIdx.x) * waves_per_block + (threadIdx.x >> 6);
+  const int64_t nwaves = (int64_t)order.blocks * waves_per_block;
   const int lane = threadIdx.x & 63;
   // The member table and the tile map stay unchanged during the launch: read through the constant
   // address space they become wave-uniform scalar loads, also after the stores of earlier tiles (the
@@ -118,54 +116,56 @@ batch_kernel(const BatchEntry<TC>* __restrict__ members, const int32_t* __restri
         a.src = a.dst;
         a.dst = t;
       }
-      const uint32_t nx = (uint32_t)a.nx, ny = (uint32_t)a.ny;
-      const uint32_t row = local / nx;
-      const int x = (int)(local - row * nx);
-      const uint32_t zz = row / ny;
-      const int y = (int)(row - zz * ny);
-      sweep_cell<S, FAM, PAT, true, true, TS, TC>(a, x, y, (int)zz);
+      const CellDivider in_row = {e->a.row.d, e->a.row.mul, e->a.row.shift};
+      const CellDivider in_plane = {e->a.plane.d, e->a.plane.mul, e->a.plane.shift};
+      const uint32_t row = in_row.quotient(local), zz = in_plane.quotient(row);
+      const int x = (int)(local - row * in_row.d);
+      const int y = (int)(row - zz * in_plane.d);
+      sweep_cell<S, FAM, PAT, true, NT, TS, TC>(a, x, y, (int)zz);
     }
   }
 }
 
 template <class TC>
-using BatchFn = void (*)(const BatchEntry<TC>*, const int32_t*, int64_t, int, int);
+using BatchFn = void (*)(const BatchEntry<TC>*, const int32_t*, int64_t, int, int, XcdOrder);
 
 template <class S, int FAM, class TS, class TC>
-void* batch_pick_pattern(int pat) {
+void* batch_pick_pattern(int pat, bool nt) {
+#define LBM_BATCH(P, NT) (void*)batch_kernel<S, FAM, P, NT, TS, TC>
   switch (pat) {
-    case LBM355_PULL: return (void*)batch_kernel<S, FAM, LBM355_PULL, TS, TC>;
-    case LBM355_AA_EVEN: return (void*)batch_kernel<S, FAM, LBM355_AA_EVEN, TS, TC>;
-    case LBM355_AA_ODD: return (void*)batch_kernel<S, FAM, LBM355_AA_ODD, TS, TC>;
+    case LBM355_PULL: return nt ? LBM_BATCH(LBM355_PULL, true) : LBM_BATCH(LBM355_PULL, false);
+    case LBM355_AA_EVEN: return nt ? LBM_BATCH(LBM355_AA_EVEN, true) : LBM_BATCH(LBM355_AA_EVEN, false);
+    case LBM355_AA_ODD: return LBM_BATCH(LBM355_AA_ODD, false);
   }
+#undef LBM_BATCH
   return nullptr;
 }
 
 template <class S, int FAM, class TC>
-void* batch_pick_store(int store, int pat) {
+void* batch_pick_store(int store, int pat, bool nt) {
   if constexpr (sizeof(TC) == 8) {
-    if (store == LBM355_F64) return batch_pick_pattern<S, FAM, double, TC>(pat);
+    if (store == LBM355_F64) return batch_pick_pattern<S, FAM, double, TC>(pat, nt);
   } else {
-    if (store == LBM355_F32) return batch_pick_pattern<S, FAM, float, TC>(pat);
-    if (store == LBM355_F16) return batch_pick_pattern<S, FAM, _Float16, TC>(pat);
+    if (store == LBM355_F32) return batch_pick_pattern<S, FAM, float, TC>(pat, nt);
+    if (store == LBM355_F16) return batch_pick_pattern<S, FAM, _Float16, TC>(pat, nt);
   }
   return nullptr;
 }
 
 template <class TC>
-void* batch_pick(const lbm355_sweep_desc* d, int pattern) {
+void* batch_pick(const lbm355_sweep_desc* d, int pattern, bool nt) {
   if (d->family == LBM355_FAMILY_MOMENT) {
-    if (d->stencil == LBM355_D2Q9) return batch_pick_store<D2Q9, LBM355_FAMILY_MOMENT, TC>(d->store_dtype, pattern);
-    if (d->stencil == LBM355_D3Q19) return batch_pick_store<D3Q19, LBM355_FAMILY_MOMENT, TC>(d->store_dtype, pattern);
-    if (d->stencil == LBM355_D3Q27) return batch_pick_store<D3Q27, LBM355_FAMILY_MOMENT, TC>(d->store_dtype, pattern);
+    if (d->stencil == LBM355_D2Q9) return batch_pick_store<D2Q9, LBM355_FAMILY_MOMENT, TC>(d->store_dtype, pattern, nt);
+    if (d->stencil == LBM355_D3Q19) return batch_pick_store<D3Q19, LBM355_FAMILY_MOMENT, TC>(d->store_dtype, pattern, nt);
+    if (d->stencil == LBM355_D3Q27) return batch_pick_store<D3Q27, LBM355_FAMILY_MOMENT, TC>(d->store_dtype, pattern, nt);
   } else if (d->family == LBM355_FAMILY_CUMULANT && d->stencil == LBM355_D3Q27) {
     if (d->flags & LBM355_FLAG_HIGHER_ORDERS_RATE1)
-      return batch_pick_store<D3Q27, FAMILY_CUMULANT_EQ3, TC>(d->store_dtype, pattern);
-    return batch_pick_store<D3Q27, LBM355_FAMILY_CUMULANT, TC>(d->store_dtype, pattern);
+      return batch_pick_store<D3Q27, FAMILY_CUMULANT_EQ3, TC>(d->store_dtype, pattern, nt);
+    return batch_pick_store<D3Q27, LBM355_FAMILY_CUMULANT, TC>(d->store_dtype, pattern, nt);
   } else if (d->family == LBM355_FAMILY_CENTRAL) {
-    if (d->stencil == LBM355_D2Q9) return batch_pick_store<D2Q9, LBM355_FAMILY_CENTRAL, TC>(d->store_dtype, pattern);
-    if (d->stencil == LBM355_D3Q19) return batch_pick_store<D3Q19, LBM355_FAMILY_CENTRAL, TC>(d->store_dtype, pattern);
-    if (d->stencil == LBM355_D3Q27) return batch_pick_store<D3Q27, LBM355_FAMILY_CENTRAL, TC>(d->store_dtype, pattern);
+    if (d->stencil == LBM355_D2Q9) return batch_pick_store<D2Q9, LBM355_FAMILY_CENTRAL, TC>(d->store_dtype, pattern, nt);
+    if (d->stencil == LBM355_D3Q19) return batch_pick_store<D3Q19, LBM355_FAMILY_CENTRAL, TC>(d->store_dtype, pattern, nt);
+    if (d->stencil == LBM355_D3Q27) return batch_pick_store<D3Q27, LBM355_FAMILY_CENTRAL, TC>(d->store_dtype, pattern, nt);
   }
   return nullptr;
 }
@@ -174,12 +174,31 @@ void* batch_pick(const lbm355_sweep_desc* d, int pattern) {
 
 using namespace lbm355;
 
+// How a batch reaches memory, by the rules of single sweeps (sweep_launch): in the caches if all its populations fit
+// half the Infinity Cache, past them if every member's cells start on lines, and else with regular accesses and
+// neighbouring tiles on one XCD.  D3Q19 TRT on MI355X, us per step, with non-temporal accesses wherever x is unshifted
+// and now: 48 ragged channels of 32..96 cells a side (1.66 GB, FP32 pull) 329 -> 289, 40 of them in FP64 500 -> 432, 16
+// of 16..40 13.9 -> 11.9; 64^3 channels: 32 FP32 pull 235 -> 214, 12 AA (239 MB) 191 -> 77.  Advancing groups of members
+// that fit the cache by several steps each gained less (1.66 GB: 307 for groups of 192 MiB).
+enum BatchAccess { BATCH_CACHED, BATCH_LINES, BATCH_SHARED };
+
+BatchAccess batch_access(const lbm355_sweep_desc* d, const void* const* src, void* const* dst, int32_t n) {
+  int64_t bytes = 0;
+  bool lines = true;
+  for (int32_t k = 0; k < n; ++k) {
+    bytes += population_bytes(&d[k], src[k] == dst[k]);
+    lines = lines && starts_lines(&d[k], src[k], dst[k]);
+  }
+  return bytes <= HALF_CACHE_BYTES ? BATCH_CACHED : lines ? BATCH_LINES : BATCH_SHARED;
+}
+
 struct lbm355_batch {
   int32_t stencil, family, store_dtype, compute_dtype, pattern_kind;  // pattern_kind: PULL or AA
   int32_t variant_flags;  // the kernel-selecting flags the members share (LBM355_FLAG_HIGHER_ORDERS_RATE1)
   int32_t nmembers;
   int64_t ntiles;
   int64_t ncells;
+  BatchAccess access;
   void* entries;          // device array of BatchEntry<TC>
   int32_t* tile_member;   // device array: member of each 64-cell tile
   int device;
@@ -227,6 +246,7 @@ int upload(const lbm355_sweep_desc* d, const void* const* src, void* const* dst,
     if (dmap) (void)hipFree(dmap);
     return berr(LBM355_ERR_LAUNCH, std::string("batch table upload failed: ") + hipGetErrorString(e));
   }
+  b->access = batch_access(d, src, dst, n);
   b->entries = dev;
   b->tile_member = (int32_t*)dmap;
   b->ntiles = tiles;
@@ -272,7 +292,7 @@ int check_members(const lbm355_sweep_desc* descs, const void* const* pdf_src, vo
     if (kind0 == LBM355_PULL && pdf_src[k] == pdf_dst[k]) return berr(LBM355_ERR_ARG, "pull needs two arrays");
     if (kind0 != LBM355_PULL && pdf_src[k] != pdf_dst[k]) return berr(LBM355_ERR_ARG, "AA needs src == dst");
   }
-  void* probe = d0.compute_dtype == LBM355_F64 ? batch_pick<double>(&d0, kind0) : batch_pick<float>(&d0, kind0);
+  void* probe = d0.compute_dtype == LBM355_F64 ? batch_pick<double>(&d0, kind0, true) : batch_pick<float>(&d0, kind0, true);
   if (!probe) return berr(LBM355_ERR_UNSUPPORTED, "no batched kernel for this stencil/family/dtype combination");
   return LBM355_OK;
 }
@@ -289,32 +309,48 @@ int check_launch(int32_t pattern_kind, int32_t step_kind, int32_t threads, int32
   return LBM355_OK;
 }
 
-// The launch of one batched step (shared by the allocating and the allocation-free entry points).
-int launch_batch(int32_t stencil, int32_t family, int32_t store_dtype, int32_t compute_dtype, int32_t pattern_kind,
-                 int32_t variant_flags, const void* entries, const int32_t* tile_member, int64_t ntiles,
-                 int32_t step_kind, int32_t threads, int32_t blocks, int32_t xcd_order, hipStream_t s) {
-  int rc = check_launch(pattern_kind, step_kind, threads, blocks);
+// What a launch needs of a batch (shared by the allocating and the allocation-free entry points).
+struct BatchLaunch {
+  int32_t stencil, family, store_dtype, compute_dtype, pattern_kind, variant_flags;
+  const void* entries;
+  const int32_t* tile_member;
+  int64_t ntiles;
+  BatchAccess access;
+};
+
+int launch_batch(const BatchLaunch& b, int32_t step_kind, int32_t threads, int32_t blocks, int32_t xcd_order,
+                 hipStream_t s) {
+  int rc = check_launch(b.pattern_kind, step_kind, threads, blocks);
   if (rc) return rc;
-  const int pattern = pattern_kind == LBM355_PULL ? LBM355_PULL : step_kind;
-  const int swap = pattern_kind == LBM355_PULL ? step_kind : 0;
+  const int pattern = b.pattern_kind == LBM355_PULL ? LBM355_PULL : step_kind;
+  const int swap = b.pattern_kind == LBM355_PULL ? step_kind : 0;
   lbm355_sweep_desc d{};
-  d.stencil = stencil;
-  d.family = family;
-  d.store_dtype = store_dtype;
-  d.flags = variant_flags;
-  void* k = compute_dtype == LBM355_F64 ? batch_pick<double>(&d, pattern) : batch_pick<float>(&d, pattern);
+  d.stencil = b.stencil;
+  d.family = b.family;
+  d.store_dtype = b.store_dtype;
+  d.flags = b.variant_flags;
+  const bool nt = b.access == BATCH_LINES;
+  void* k = b.compute_dtype == LBM355_F64 ? batch_pick<double>(&d, pattern, nt) : batch_pick<float>(&d, pattern, nt);
   if (!k) return berr(LBM355_ERR_UNSUPPORTED, "no batched kernel");
-  const int64_t max_blocks = (ntiles * 64 + threads - 1) / threads;
+  const int64_t max_blocks = (b.ntiles * 64 + threads - 1) / threads;
   const int grid = (int)(blocks < max_blocks ? blocks : max_blocks);
-  if (compute_dtype == LBM355_F64)
-    hipLaunchKernelGGL((BatchFn<double>)k, dim3(grid), dim3(threads), 0, s, (const BatchEntry<double>*)entries,
-                       tile_member, ntiles, swap, xcd_order);
+  const bool runs = b.access == BATCH_CACHED || (xcd_order && grid % 8 == 0);
+  const int chunk = runs ? grid / 8 : nt ? 1 : SHARED_LINES_CHUNK;
+  const XcdOrder order = XcdOrder::of(grid, chunk);
+  if (b.compute_dtype == LBM355_F64)
+    hipLaunchKernelGGL((BatchFn<double>)k, dim3(grid), dim3(threads), 0, s, (const BatchEntry<double>*)b.entries,
+                       b.tile_member, b.ntiles, swap, threads / 64, order);
   else
-    hipLaunchKernelGGL((BatchFn<float>)k, dim3(grid), dim3(threads), 0, s, (const BatchEntry<float>*)entries,
-                       tile_member, ntiles, swap, xcd_order);
+    hipLaunchKernelGGL((BatchFn<float>)k, dim3(grid), dim3(threads), 0, s, (const BatchEntry<float>*)b.entries,
+                       b.tile_member, b.ntiles, swap, threads / 64, order);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return berr(LBM355_ERR_LAUNCH, std::string("launch failed: ") + hipGetErrorString(e));
   return LBM355_OK;
+}
+
+BatchLaunch launch_of(const lbm355_batch* b) {
+  return {b->stencil, b->family, b->store_dtype, b->compute_dtype, b->pattern_kind, b->variant_flags, b->entries,
+          b->tile_member, b->ntiles, b->access};
 }
 }  // namespace
 
@@ -350,9 +386,7 @@ int lbm355_batch_create(const lbm355_sweep_desc* descs, const void* const* pdf_s
 int lbm355_batch_sweep(const lbm355_batch* b, int32_t step_kind, int32_t threads, int32_t blocks,
                        int32_t xcd_order, void* stream) {
   if (!b) return berr(LBM355_ERR_ARG, "batch is NULL");
-  return launch_batch(b->stencil, b->family, b->store_dtype, b->compute_dtype, b->pattern_kind, b->variant_flags,
-                      b->entries, b->tile_member, b->ntiles, step_kind, threads, blocks, xcd_order,
-                      (hipStream_t)stream);
+  return launch_batch(launch_of(b), step_kind, threads, blocks, xcd_order, (hipStream_t)stream);
 }
 
 int lbm355_batch_info(const lbm355_batch* b, int64_t* n_tiles, int64_t* n_cells) {
@@ -447,9 +481,10 @@ int static_step(const lbm355_sweep_desc* descs, const void* const* src, void* co
   e = hipGetLastError();
   if (e != hipSuccess) return berr(LBM355_ERR_LAUNCH, std::string("tile-map launch failed: ") + hipGetErrorString(e));
   const lbm355_sweep_desc& d0 = descs[0];
-  return launch_batch(d0.stencil, d0.family, d0.store_dtype, d0.compute_dtype, kind,
-                      d0.flags & LBM355_FLAG_HIGHER_ORDERS_RATE1, dev_table, dev_map, tiles,
-                      step_kind, threads, blocks, xcd_order, s);
+  const BatchLaunch l = {d0.stencil, d0.family, d0.store_dtype, d0.compute_dtype, kind,
+                         d0.flags & LBM355_FLAG_HIGHER_ORDERS_RATE1, dev_table, dev_map, tiles,
+                         batch_access(descs, src, dst, n)};
+  return launch_batch(l, step_kind, threads, blocks, xcd_order, s);
 }
 }  // namespace
 
