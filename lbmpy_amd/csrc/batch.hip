@@ -174,22 +174,26 @@ void* batch_pick(const lbm355_sweep_desc* d, int pattern, bool nt) {
 
 using namespace lbm355;
 
-// How a batch reaches memory, by the rules of single sweeps (sweep_launch): in the caches if all its populations fit
-// half the Infinity Cache, past them if every member's cells start on lines, and else with regular accesses and
-// neighbouring tiles on one XCD.  D3Q19 TRT on MI355X, us per step, with non-temporal accesses wherever x is unshifted
-// and now: 48 ragged channels of 32..96 cells a side (1.66 GB, FP32 pull) 329 -> 289, 40 of them in FP64 500 -> 432, 16
-// of 16..40 13.9 -> 11.9; 64^3 channels: 32 FP32 pull 235 -> 214, 12 AA (239 MB) 191 -> 77.  Advancing groups of members
-// that fit the cache by several steps each gained less (1.66 GB: 307 for groups of 192 MiB).
-enum BatchAccess { BATCH_CACHED, BATCH_LINES, BATCH_SHARED };
+// How a batch reaches memory, by the rules of single sweeps (sweep_launch) for the populations of all members: in the
+// caches if they fit half the Infinity Cache (64^3 AA, 239 MB: 98 us so, 78 past it), past them if every member's cells
+// start on lines, and else with regular accesses and neighbouring tiles on one XCD, in turns (meets_cached) every other
+// step backwards.  D3Q19 TRT on MI355X, us per step, with non-temporal accesses wherever x is unshifted and now: 48
+// ragged channels of 32..96 cells a side (1.66 GB, FP32 pull) 329 -> 289, 40 of them in FP64 500 -> 432, 16 of 16..40
+// 13.9 -> 11.9; 64^3 channels: 32 FP32 pull 235 -> 215, 12 AA 191 -> 77; 40 of 61x63x67 FP16 AA 267 -> 224.  Advancing
+// groups of members that fit the cache by several steps each gained less (1.66 GB: 307 for groups of 192 MiB).
+enum BatchAccess { BATCH_CACHED, BATCH_LINES, BATCH_SHARED, BATCH_TURNS };
 
 BatchAccess batch_access(const lbm355_sweep_desc* d, const void* const* src, void* const* dst, int32_t n) {
   int64_t bytes = 0;
   bool lines = true;
+  const bool in_place = src[0] == dst[0];     // of all members alike (check_members)
   for (int32_t k = 0; k < n; ++k) {
-    bytes += population_bytes(&d[k], src[k] == dst[k]);
+    bytes += population_bytes(&d[k], in_place);
     lines = lines && starts_lines(&d[k], src[k], dst[k]);
   }
-  return bytes <= HALF_CACHE_BYTES ? BATCH_CACHED : lines ? BATCH_LINES : BATCH_SHARED;
+  if (bytes <= HALF_CACHE_BYTES) return BATCH_CACHED;
+  if (lines) return BATCH_LINES;
+  return meets_cached(bytes, in_place) ? BATCH_TURNS : BATCH_SHARED;
 }
 
 struct lbm355_batch {
@@ -336,7 +340,7 @@ int launch_batch(const BatchLaunch& b, int32_t step_kind, int32_t threads, int32
   const int grid = (int)(blocks < max_blocks ? blocks : max_blocks);
   const bool runs = b.access == BATCH_CACHED || (xcd_order && grid % 8 == 0);
   const int chunk = runs ? grid / 8 : nt ? 1 : SHARED_LINES_CHUNK;
-  const XcdOrder order = XcdOrder::of(grid, chunk);
+  const XcdOrder order = XcdOrder::of(grid, chunk, b.access == BATCH_TURNS && (swap || step_kind == LBM355_AA_EVEN));
   if (b.compute_dtype == LBM355_F64)
     hipLaunchKernelGGL((BatchFn<double>)k, dim3(grid), dim3(threads), 0, s, (const BatchEntry<double>*)b.entries,
                        b.tile_member, b.ntiles, swap, threads / 64, order);

@@ -193,15 +193,17 @@ struct CellDivider {
 
 // Consecutive workgroups go to the 8 XCDs in turn, each with an L2 of its own.  XcdOrder renumbers them so that runs of
 // `chunk` neighbouring block numbers share an XCD: within every group of 8 chunk blocks, the blocks of one XCD take
-// one run.  The blocks after the last whole group, and all of them with chunk <= 1, keep their numbers.
+// one run.  The blocks after the last whole group, and all of them with chunk <= 1, keep their numbers.  `backwards`: from
+// the last block number to the first.
 struct XcdOrder {
-  uint32_t blocks, chunk;
+  uint32_t blocks, chunk, backwards;
   CellDivider group;
-  __host__ __device__ static XcdOrder of(uint32_t blocks, uint32_t chunk) {
+  __host__ __device__ static XcdOrder of(uint32_t blocks, uint32_t chunk, bool backwards = false) {
     if (chunk < 1) chunk = 1;
-    return {blocks, chunk, CellDivider::of(8 * chunk)};
+    return {blocks, chunk, backwards, CellDivider::of(8 * chunk)};
   }
   __host__ __device__ __forceinline__ uint32_t number(uint32_t block) const {
+    if (backwards) block = blocks - 1 - block;
     const uint32_t first = group.quotient(block) * group.d, k = block - first;
     return first + group.d > blocks ? block : first + (k & 7) * chunk + (k >> 3);
   }
@@ -234,7 +236,7 @@ struct SweepArgs {
   uint32_t seed;              // stochastic FP16 rounding: this launch's seed
   CellDivider row, plane;     // division by nx and by ny (thread_cell)
   XcdOrder order;             // of the blocks (thread_cell)
-  uint32_t block;             // threads per block: blockDim.x would be a load of its own, waited for before the first
+  uint32_t block;             // threads per block (thread_cell)
 };
 
 // What a collision hands back to the cell beyond the populations: the Smagorinsky shear rate and Pi

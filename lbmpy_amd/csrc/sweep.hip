@@ -451,8 +451,7 @@ int validate(const lbm355_sweep_desc* d) {
 template <class TC>
 int launch_sweep(const lbm355_sweep_desc* d, const void* src, void* dst, void* rho, void* u, hipStream_t s) {
   if (table_pattern(d->pattern)) return lbm355_launch_sweep_eso(d, src, dst, rho, u, s);
-  bool walls = false;
-  for (int a = 0; a < stencil_d(d->stencil); ++a) walls |= d->face[a] == LBM355_FACE_NOSLIP;
+  const bool walls = has_walls(d);
   size_t lds = 0;
   const bool odd = d->pattern == LBM355_AA_ODD;
   const SweepLaunch l = sweep_launch(d, src, dst, use_rowlds(d, &lds), !odd, !odd);

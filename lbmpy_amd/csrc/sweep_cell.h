@@ -353,10 +353,12 @@ enum AccessMode { ACCESS_ROWS, ACCESS_WAVES, ACCESS_LINES, ACCESS_CACHED };
 // The cell of this thread, or false beyond the last cell.  Threads number the cells consecutively over rows and
 // planes, so that wavefronts are full whatever nx is; with ACCESS_WAVES, blocks take up to 256 cells of one row, and y
 // and z stay in scalar registers (256^3 FP32 AA even: 593 us, 616 us with numbered cells; FP16 storage 315 and 329).
+// The block size is an argument: blockDim.x is a load of its own, waited for before the first address.  (The streamed
+// rows keep it: 256^3 AA is 0.4% slower without that wait.)
 template <int MODE, class TC>
 __device__ __forceinline__ bool thread_cell(const SweepArgs<TC>& a, int& x, int& y, int& z) {
   if constexpr (MODE == ACCESS_WAVES) {
-    x = blockIdx.x * a.block + threadIdx.x;
+    x = blockIdx.x * blockDim.x + threadIdx.x;
     y = blockIdx.y;
     z = blockIdx.z;
     return x < a.nx;
@@ -393,26 +395,51 @@ inline bool starts_lines(const lbm355_sweep_desc* d, const void* src, const void
 //   regular accesses, 640 with runs of 16 blocks per XCD), FP16 250x200x180 252 -> 170.
 // - Otherwise two wavefronts share most lines, and non-temporal accesses move those twice; regular ones, with
 //   neighbouring blocks on one XCD, do not: 256^3 with ghost layers 947 -> 709 (809 without the runs), 251x255x253
-//   793 -> 684, FP64 131x117x101 143 -> 117.
+//   793 -> 684, FP64 131x117x101 143 -> 117.  Every other sweep backwards takes them to 646 and 102 (meets_cached).
 // Full wavefronts whatever nx is matter most for short rows: D3Q19 TRT 35x148x256 84 -> 28.
 constexpr uint32_t SHARED_LINES_CHUNK = 16;
 constexpr int64_t SMALL_CELLS = 1 << 18;   // below: blocks of one wavefront, to spread over the 256 CUs
 
 // Whether the populations' bytes fit the 256 MiB Infinity Cache to a gain.  In place in FP32 or FP64 they may fill it:
 // at 128^3 (216 MiB) regular accesses win also for a program that takes three such arrays in turn (82 -> 71 us, one
-// array 57).  Two arrays, FP16 storage and the learned closure lose more to such turns than they gain alone (pull D3Q19
-// 128x128x80, 253 MB: 36.7 -> 29.9 us for one pair of arrays, 42.5 for three in turn; FP16 192x128x128, 162 MiB: 54.7
-// -> 49.5, 63.5; closure 128^3: 107 -> 99, 116): they may fill half of it, where they do not (closure 128x96x96: 67 ->
-// 61, 66).
+// array 57; learned closure 107 -> 79, three in turn 106 -> 96).  Two arrays and FP16 storage lose more to such turns
+// than they gain alone (pull D3Q19 128x128x80, 253 MB: 36.7 -> 29.9 us for one pair of arrays, 42.5 for three in turn;
+// FP16 192x128x128, 162 MiB: 54.7 -> 49.5, 63.5): they may fill half of it, where they do not.
 inline int64_t population_bytes(const lbm355_sweep_desc* d, bool in_place) {
   const int64_t es = d->store_dtype == LBM355_F64 ? 8 : (d->store_dtype == LBM355_F32 ? 4 : 2);
   const int q = d->stencil == LBM355_D2Q9 ? 9 : (d->stencil == LBM355_D3Q19 ? 19 : 27);
   return (in_place ? 1 : 2) * q * es * d->nx * d->ny * d->nz;
 }
 constexpr int64_t HALF_CACHE_BYTES = int64_t(128) << 20;
-inline bool fits_cache(const lbm355_sweep_desc* d, bool in_place) {
-  const bool half = !in_place || d->store_dtype == LBM355_F16 || (d->flags & LBM355_FLAG_LEARNED_CLOSURE);
-  return population_bytes(d, in_place) <= (half ? HALF_CACHE_BYTES : 2 * HALF_CACHE_BYTES);
+inline bool fits_cache(int64_t bytes, int store, bool in_place) {
+  return bytes <= (!in_place || store == LBM355_F16 ? HALF_CACHE_BYTES : 2 * HALF_CACHE_BYTES);
+}
+
+// Larger populations still meet a part of themselves in the cache, what the sweep before reached last, if every other
+// sweep goes backwards: the even one of an in-place pattern; of two arrays, the one from the lower address.  us per
+// launch forwards and so, one array (three in turn, two sweeps on each): D3Q27 cumulant AA FP64 131x117x101 117 (127)
+// and 102 (111), FP32 181x175x153 222 (223) and 177 (202), 251x255x253 687 (688) and 646 (666), D3Q19 TRT AA 192x180x144
+// with ghost layers and walls 152 (155) and 121 (135), pull 192x160x144 with ghost layers, 672 MB, 165 (164) and 150
+// (159).  Two arrays of 1.8 GB lose 1%.
+inline bool backwards_sweep(int pattern, const void* src, const void* dst) {
+  switch (pattern) {
+    case LBM355_AA_EVEN: case LBM355_ESOTWIST_EVEN: case LBM355_ESOPULL_EVEN: case LBM355_ESOPUSH_EVEN: return true;
+  }
+  return src != dst && (uintptr_t)src < (uintptr_t)dst;
+}
+inline bool meets_cached(int64_t bytes, bool in_place) { return in_place || bytes <= 8 * HALF_CACHE_BYTES; }
+// Whether that is worth regular accesses where the lines would allow non-temporal ones: D3Q27 cumulant AA FP32 160^3,
+// 442 MB, 151 (151) streamed and 132 (151) so, 192^3, 764 MB, 276 (276) and 248 (266), but 224^3, 1.2 GB, 438 (437) and
+// 433 (444); FP64 128^3 161 (162) and 136 (158); EsoTwist FP32 150x150x160 147 (151) and 125 (135).  With walls arrays in
+// turn lose (D3Q19 TRT 200x200x160 156 (156) and 152 (165)), FP16 too (200^3 146 (145) and 134 (153)), and two arrays
+// gain nothing (D3Q19 TRT pull 160^3 119 (119) and 117 (118)).
+inline bool cached_anyway(int64_t bytes, int store, bool in_place, bool walls) {
+  return in_place && !walls && store != LBM355_F16 && bytes <= 6 * HALF_CACHE_BYTES;
+}
+inline bool has_walls(const lbm355_sweep_desc* d) {
+  for (int a = 0; a < (d->stencil == LBM355_D2Q9 ? 2 : 3); ++a)
+    if (d->face[a] == LBM355_FACE_NOSLIP) return true;
+  return false;
 }
 
 struct SweepLaunch {
@@ -425,8 +452,10 @@ struct SweepLaunch {
 // row_kernel, waves_kernel, lines_kernel: whether the caller has a kernel of that mode for this sweep.
 inline SweepLaunch sweep_launch(const lbm355_sweep_desc* d, const void* src, const void* dst, bool row_kernel,
                                 bool waves_kernel, bool lines_kernel) {
-  const bool fits = fits_cache(d, src == dst), half = population_bytes(d, src == dst) <= HALF_CACHE_BYTES;
-  const bool lines = !fits && starts_lines(d, src, dst);
+  const bool in_place = src == dst;
+  const int64_t bytes = population_bytes(d, in_place);
+  const bool fits = fits_cache(bytes, d->store_dtype, in_place), half = bytes <= HALF_CACHE_BYTES;
+  const bool lines = !fits && !cached_anyway(bytes, d->store_dtype, in_place, has_walls(d)) && starts_lines(d, src, dst);
   if (row_kernel && lines) return {ACCESS_ROWS, dim3(1, d->ny, d->nz), dim3(d->nx), XcdOrder::of(1, 1), half};
   if (waves_kernel && lines && d->nx % 64 == 0) {
     const unsigned bx = d->nx < 256 ? d->nx : 256;
@@ -436,7 +465,9 @@ inline SweepLaunch sweep_launch(const lbm355_sweep_desc* d, const void* src, con
   const unsigned bx = cells < SMALL_CELLS ? 64 : 256;
   const unsigned blocks = (unsigned)((cells + bx - 1) / bx);
   if (lines_kernel && lines) return {ACCESS_LINES, dim3(blocks), dim3(bx), XcdOrder::of(blocks, 1), half};
-  return {ACCESS_CACHED, dim3(blocks), dim3(bx), XcdOrder::of(blocks, fits ? blocks / 8 : SHARED_LINES_CHUNK), half};
+  const bool backwards = !fits && meets_cached(bytes, in_place) && backwards_sweep(d->pattern, src, dst);
+  const unsigned chunk = fits ? blocks / 8 : SHARED_LINES_CHUNK;
+  return {ACCESS_CACHED, dim3(blocks), dim3(bx), XcdOrder::of(blocks, chunk, backwards), half};
 }
 
 // Kernel arguments from a public descriptor (include/lbm355.h).

@@ -15,7 +15,7 @@ __global__ void __launch_bounds__(MODE == ACCESS_ROWS ? 512 : 256) sweep_kernel(
     if (!thread_cell<MODE>(a, x, y, z)) return;
     sweep_cell<S, FAM, PAT, WALLS, MODE != ACCESS_CACHED, TS, TC>(a, x, y, z);
   } else {
-    const int x = threadIdx.x;
+    const int x = blockIdx.x * blockDim.x + threadIdx.x;
     // The block spans one whole periodic row (blockDim.x == nx).  The +-1 x-shifts of pull / AA-odd
     // streaming go through LDS, so every global access is an aligned, contiguous, non-temporal one.
     constexpr int Q = S::Q, D = S::D;
