@@ -298,6 +298,11 @@ typedef struct lbm355_boundary_desc {
 int lbm355_boundary_links(const lbm355_boundary_desc* desc, void* pdf, const int32_t* links, int64_t n_links,
                           double* link_data, void* stream);
 
+/* lbm355_boundary_links for n_groups conditions on one array, in this order (host arrays of descriptors, pointers and
+ * counts); consecutive NoSlip and UBB groups, whose links are independent, share a launch. */
+int lbm355_boundary_groups(const lbm355_boundary_desc* descs, int32_t n_groups, void* pdf, const int32_t* const* links,
+                           const int64_t* n_links, double* const* link_data, void* stream);
+
 /* ---- Ghost-layer periodicity -----------------------------------------------------------------------
  * For sweeps whose faces are LBM355_FACE_GHOST (lbmpy's own kernels never wrap): the copies of lbmpy's
  * LBMPeriodicityHandling (advanced_streaming/communication.py:21-126), each source slice of

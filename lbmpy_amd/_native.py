@@ -70,7 +70,8 @@ EXPORTED = ("lbm355_sweep", "lbm355_table_elements", "lbm355_noslip_links", "lbm
             "lbm355_batch_info", "lbm355_batch_destroy", "lbm355_batch_sweep_static", "lbm355_closure_params_size",
             "lbm355_closure_master_size", "lbm355_closure_features", "lbm355_closure_forward",
             "lbm355_closure_train_step", "lbm355_closure_adam", "lbm355_closure_workspace_floats",
-            "lbm355_closure_gradient", "lbm355_closure_train_epoch", "lbm355_boundary_links", "lbm355_copy_boxes",
+            "lbm355_closure_gradient", "lbm355_closure_train_epoch", "lbm355_boundary_links", "lbm355_boundary_groups",
+            "lbm355_copy_boxes",
             "lbm355_pattern_access", "lbm355_get_strain_rate", "lbm355_plane_copy", "lbm355_valu_probe",
             "lbm355_source_hash")
 
@@ -149,6 +150,8 @@ def load(path=None):
     lib.lbm355_boundary_links.argtypes = [ctypes.POINTER(BoundaryDesc), c_void_p, c_void_p, c_int64, c_void_p,
                                           c_void_p]
     lib.lbm355_boundary_links.restype = c_int32
+    lib.lbm355_boundary_groups.argtypes = [c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]
+    lib.lbm355_boundary_groups.restype = c_int32
     lib.lbm355_get_strain_rate.argtypes = [ctypes.POINTER(SweepDesc), c_void_p, c_void_p, c_void_p, c_double, c_int32,
                                            c_void_p]
     lib.lbm355_get_strain_rate.restype = c_int32

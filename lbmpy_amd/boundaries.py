@@ -542,9 +542,23 @@ class LatticeBoltzmannBoundaryHandling:
             raise TypeError("boundaries run on GPU tensors of float64, float32 or float16")
         lib = nat.load()
         faces = self._faces
-        for group in groups:
+        n = len(groups)
+        descs = (nat.BoundaryDesc * n)()
+        linkp, datap, counts = (ctypes.c_void_p * n)(), (ctypes.c_void_p * n)(), (ctypes.c_int64 * n)()
+        pending = 0
+
+        def launch(end):
+            nonlocal pending
+            at, pending = pending, end
+            nat.check(lib.lbm355_boundary_groups(ctypes.byref(descs, at * ctypes.sizeof(nat.BoundaryDesc)), end - at,
+                                                 ctypes.c_void_p(pdf.data_ptr()), ctypes.byref(linkp, 8 * at),
+                                                 ctypes.byref(counts, 8 * at), ctypes.byref(datap, 8 * at),
+                                                 nat.current_stream_handle()))
+
+        for k, group in enumerate(groups):
             obj, links, vel, ready = group
-            d = nat.BoundaryDesc()
+            linkp[k], datap[k], counts[k] = links.data_ptr(), vel.data_ptr() if vel is not None else None, links.shape[0]
+            d = descs[k]
             d.stencil = nat.STENCIL_NAMES[m.stencil.name]
             d.pattern = int(pattern_code)
             d.store_dtype = dtypes[pdf.dtype]
@@ -581,6 +595,7 @@ class LatticeBoltzmannBoundaryHandling:
                 for ax, v in enumerate(obj.normal_direction):
                     d.normal[ax] = int(v)
                 if not ready:
+                    launch(k)
                     # the state starts from the populations present now (read through the same accessor)
                     d.kind = nat.BC_OUTFLOW_INIT
                     nat.check(lib.lbm355_boundary_links(ctypes.byref(d), ctypes.c_void_p(pdf.data_ptr()),
@@ -601,10 +616,7 @@ class LatticeBoltzmannBoundaryHandling:
                         d.flags |= nat.FLAG_EQ_SHIFT
                     for ax in range(D):
                         d.force[ax] = float(fm.force[ax])
-            nat.check(lib.lbm355_boundary_links(ctypes.byref(d), ctypes.c_void_p(pdf.data_ptr()),
-                                                ctypes.c_void_p(links.data_ptr()), links.shape[0],
-                                                ctypes.c_void_p(vel.data_ptr() if vel is not None else 0),
-                                                nat.current_stream_handle()))
+        launch(n)
 
     def __call__(self, prev_timestep=None, **kwargs):
         """lbmpy's form: applies the boundaries to the data handling's PDF array after the kernel that ran at
