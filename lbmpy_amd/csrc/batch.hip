@@ -178,7 +178,7 @@ using namespace lbm355;
 // caches if they fit half the Infinity Cache (64^3 AA, 239 MB: 98 us so, 78 past it), past them if every member's cells
 // start on lines, and else with regular accesses and neighbouring tiles on one XCD, in turns (meets_cached) every other
 // step backwards.  D3Q19 TRT on MI355X, us per step, with non-temporal accesses wherever x is unshifted and now: 48
-// ragged channels of 32..96 cells a side (1.66 GB, FP32 pull) 329 -> 289, 40 of them in FP64 500 -> 432, 16 of 16..40
+// channels of mixed sizes, 32..96 cells a side (1.66 GB, FP32 pull) 329 -> 289, 40 of them in FP64 500 -> 432, 16 of 16..40
 // 13.9 -> 11.9; 64^3 channels: 32 FP32 pull 235 -> 215, 12 AA 191 -> 77; 40 of 61x63x67 FP16 AA 267 -> 224.  Advancing
 // groups of members that fit the cache by several steps each gained less (1.66 GB: 307 for groups of 192 MiB).
 enum BatchAccess { BATCH_CACHED, BATCH_LINES, BATCH_SHARED, BATCH_TURNS };
