@@ -51,9 +51,8 @@ __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float(((uin
 __device__ __forceinline__ float softplus(float o) { return o > 20.f ? o : log1pf(expf(o)); }
 __device__ __forceinline__ float sigmoid(float o) { return 1.f / (1.f + expf(-o)); }
 
-// raw features from the non-equilibrium second moments Pi_neq (xx, yy, zz, xy, xz, yz) and rho
-__device__ __forceinline__ void closure_features(const float (&p)[6], float rho, float (&x)[CLOSURE_IN]) {
-  const float ir = recip(rho);
+// raw features from the non-equilibrium second moments Pi_neq (xx, yy, zz, xy, xz, yz) and 1 / rho
+__device__ __forceinline__ void closure_features(const float (&p)[6], float ir, float (&x)[CLOSURE_IN]) {
   const float q[6] = {p[0] * ir, p[1] * ir, p[2] * ir, p[3] * ir, p[4] * ir, p[5] * ir};
   const float qq = q[0] * q[0] + q[1] * q[1] + q[2] * q[2] + 2.f * (q[3] * q[3] + q[4] * q[4] + q[5] * q[5]);
   // tr(q^3) of the symmetric matrix [[xx, xy, xz], [xy, yy, yz], [xz, yz, zz]]
@@ -62,25 +61,20 @@ __device__ __forceinline__ void closure_features(const float (&p)[6], float rho,
                    6.f * q[3] * q[4] * q[5];
 #pragma unroll
   for (int i = 0; i < 6; ++i) x[i] = q[i];
-  x[6] = __builtin_amdgcn_sqrtf(2.f * qq);
+  x[6] = sqrtf(2.f * qq);
   x[7] = q[0] + q[1] + q[2];
   x[8] = qq;
   x[9] = t3;
 }
 
-// tanh in FP32 for the hidden layers: 1 - 2 / (1 + e) with e = exp(2x) from the hardware base-2 exponential and
-// reciprocal (e = inf and 0 give +-1); absolute error about 2e-7, far below the BF16 step of the activations that the
-// next layer reads.  Three plain instructions and two transcendental ones; each cell takes 64 of them.
+// tanh in FP32 for the hidden layers, of training and evaluation alike: sign(x) (1 - e) / (1 + e) with e = exp(-2|x|) from
+// the hardware base-2 exponential and reciprocal.  1 - e is exact inside the multiply-add.  Over [-6, 6] the error is
+// 1.3e-7 at most and 3.1e-8 on average, below 2e-8 next to 0 (1 - 2 / (1 + exp(2x)), an instruction less, has 2.2e-7,
+// 3.8e-8 and 1.4e-7).  Four plain instructions and two transcendental ones; each cell takes 64 of them.
 __device__ __forceinline__ float tanh_fast(float x) {
-  const float e = __builtin_amdgcn_exp2f(2.885390081777927f * x);   // 2 log2(e) x
-  return __builtin_fmaf(-2.f, __builtin_amdgcn_rcpf(1.f + e), 1.f);
-}
-
-// The same as an exactly odd function, sign(x) (1 - e) / (1 + e) with e = exp(-2|x|): two instructions more, which
-// training, bound by latency, does not notice.
-__device__ __forceinline__ float tanh_odd(float x) {
-  const float e = __builtin_amdgcn_exp2f(-2.885390081777927f * fabsf(x));
-  return copysignf((1.f - e) * __builtin_amdgcn_rcpf(1.f + e), x);
+  const float e = __builtin_amdgcn_exp2f(-2.885390081777927f * fabsf(x));   // 2 log2(e) |x|
+  const float r = __builtin_amdgcn_rcpf(1.f + e);
+  return copysignf(__builtin_fmaf(-e, r, r), x);
 }
 
 // A fragment (4 BF16) of a [32 x K] row-major BF16 matrix for K block kb
@@ -101,7 +95,6 @@ __device__ __forceinline__ int c_row(int v, int lane) { return 8 * (v >> 2) + 4 
 // Wave-collective forward pass for the 64 cells of a wavefront (every lane must take part).
 // x: this lane's raw features.  Returns this lane's output o.  If h1/h2 are given, the tanh
 // activations of both cell blocks c = 0, 1 are kept in C layout (h[c][v]) for the backward pass.
-template <bool TRAINING = false>
 __device__ __forceinline__ float mlp_forward_wave(const ClosureParams* __restrict__ P, const float (&x)[CLOSURE_IN],
                                                   float (*h1)[16], float (*h2)[16]) {
   const int lane = threadIdx.x & 63;
@@ -147,7 +140,7 @@ __device__ __forceinline__ float mlp_forward_wave(const ClosureParams* __restric
     v4s hb[4];
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      const float h = TRAINING ? tanh_odd(acc[v]) : tanh_fast(acc[v]);
+      const float h = tanh_fast(acc[v]);
       if (h1) h1[c][v] = h;
       hb[v >> 2][v & 3] = (short)f2bf(h);
     }
@@ -159,7 +152,7 @@ __device__ __forceinline__ float mlp_forward_wave(const ClosureParams* __restric
     float part = 0.f;
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      const float h = TRAINING ? tanh_odd(acc2[v]) : tanh_fast(acc2[v]);
+      const float h = tanh_fast(acc2[v]);
       if (h2) h2[c][v] = h;
       part += bf2f(P->w3[c_row(v, lane)]) * h;
     }
@@ -169,15 +162,26 @@ __device__ __forceinline__ float mlp_forward_wave(const ClosureParams* __restric
   return out;
 }
 
+// softplus(o) = max(o, 0) + log(1 + e), e = exp(-|o|), for the sweep, which needs it once per cell: the hardware's base-2
+// functions, with the remainder of |o| log2(e) put back into e and the remainder of 1 + e into the logarithm, so that small
+// viscosities keep their relative accuracy.  Largest relative error 2.7e-7 over [-17, -6], 1.4e-7 below and 2.3e-7 above
+// (log1pf(expf(o)): 8.7e-7, 2.7e-6 and 5.0e-7; log(1 + e) alone is 0 below -17).
+__device__ __forceinline__ float softplus_sweep(float o) {
+  const float a = fminf(fabsf(o), 104.f);   // exp(-104) is 0
+  const float h = -1.4426950216293335f * a;
+  const float l = __builtin_fmaf(-1.4426950216293335f, a, -h) - 1.9259629911e-8f * a;
+  float e = __builtin_amdgcn_exp2f(h);
+  e = __builtin_fmaf(e, 0.6931471805599453f * l, e);
+  const float u = 1.f + e, c = e - (u - 1.f);
+  const float base = o < 0.f ? 0.f : o;     // NaN stays NaN
+  return __builtin_fmaf(__builtin_amdgcn_logf(u), 0.6931471805599453f, c * __builtin_amdgcn_rcpf(u)) + base;
+}
+
 // shear relaxation rate from the network output: nu_t = nu_scale softplus(o) - nu_shift added to the
-// molecular viscosity, relaxation time at least 0.5 + 3e-6
+// molecular viscosity, relaxation time at least 0.5 + 3e-6 (and at most 1e30, where recip still holds)
 __device__ __forceinline__ float closure_omega(const ClosureParams* __restrict__ P, float o, float omega0) {
-  // softplus(o) = max(o, 0) + log(1 + exp(-|o|)) with the hardware's base-2 functions: absolute error below 2e-7, which
-  // nu_scale makes small against the rounding of tau
-  const float e = __builtin_amdgcn_exp2f(-1.4426950408889634f * fabsf(o));
-  const float sp = __builtin_fmaf(0.6931471805599453f, __builtin_amdgcn_logf(1.f + e), fmaxf(o, 0.f));
-  const float tau = recip(omega0) + 3.f * (P->nu_scale * sp - P->nu_shift);
-  return recip(fmaxf(tau, 0.500003f));
+  const float tau = 1.f / omega0 + 3.f * (P->nu_scale * softplus_sweep(o) - P->nu_shift);
+  return recip(fminf(fmaxf(tau, 0.500003f), 1e30f));
 }
 
 }  // namespace lbm355

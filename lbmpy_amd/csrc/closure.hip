@@ -20,7 +20,7 @@ __global__ void __launch_bounds__(256) features_kernel(const float* __restrict__
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     const float p[6] = {pi6[6 * i], pi6[6 * i + 1], pi6[6 * i + 2], pi6[6 * i + 3], pi6[6 * i + 4], pi6[6 * i + 5]};
     float f[CLOSURE_IN];
-    closure_features(p, rho[i], f);
+    closure_features(p, 1.f / rho[i], f);
 #pragma unroll
     for (int k = 0; k < CLOSURE_IN; ++k) x[CLOSURE_IN * i + k] = f[k];
   }
@@ -115,7 +115,7 @@ __global__ void __launch_bounds__(64 * TRAIN_WAVES) train_kernel(const ClosurePa
     for (int k = 0; k < CLOSURE_IN; ++k) x[k] = valid ? X[CLOSURE_IN * row + k] : 0.f;
     const float y = valid ? Y[row] : 0.f;
     float h1[2][16], h2[2][16];
-    const float o = mlp_forward_wave<true>(P, x, h1, h2);
+    const float o = mlp_forward_wave(P, x, h1, h2);
     const float diff = softplus(o) - y;
     const float g = valid ? 2.f * inv_n * diff * sigmoid(o) : 0.f;
     lsum += valid ? diff * diff : 0.f;

@@ -302,7 +302,7 @@ __device__ __forceinline__ void collide_cumulant_d3q27(T (&f)[27], const SweepAr
       const ClosureParams* P = reinterpret_cast<const ClosureParams*>(a.closure);
       const float p6[6] = {pxx, pyy, pzz, pxy, pxz, pyz};
       float feat[CLOSURE_IN];
-      closure_features(p6, rho, feat);
+      closure_features(p6, recip(rho), feat);
       w = closure_omega(P, mlp_forward_wave(P, feat, nullptr, nullptr), a.omega_shear);
     }
     rs[0] = rs[1] = rs[2] = rs[3] = rs[4] = w;
