@@ -1,0 +1,85 @@
+"""The macroscopic getter writes its outputs directly only where every element written is its own."""
+import pytest
+import torch
+
+from lbmpy_amd.macroscopic_value_kernels import _own_memory
+
+SHAPE = (6, 5, 4)
+
+
+def _pdfs(q=19, extra=0):
+    return torch.zeros((q + extra,) + SHAPE[::-1]).permute(3, 2, 1, 0)
+
+
+def _c(*shape):
+    return torch.zeros(shape)
+
+
+def _f(*shape):
+    return torch.zeros(shape[::-1]).permute(*reversed(range(len(shape))))
+
+
+def test_separate_fields():
+    for make in (_c, _f):
+        assert _own_memory(_pdfs(), [make(*SHAPE), make(*SHAPE)], make(*SHAPE, 3))
+        assert _own_memory(_pdfs(), [], make(*SHAPE, 3)) and _own_memory(_pdfs(), [make(*SHAPE)], None)
+    one = torch.zeros(1, 1, 1)
+    assert _own_memory(torch.zeros(1, 1, 1, 19), [one], None)
+
+
+def test_interleaved_components_are_separate():
+    cell = _c(*SHAPE, 4)                       # [x, y, z][rho, u]
+    assert _own_memory(_pdfs(), [cell[..., 0]], cell[..., 1:])
+    assert _own_memory(_pdfs(), [cell[..., 3]], cell[..., :3])
+    plane = _f(*SHAPE, 5)                      # one x-fastest plane per component
+    assert _own_memory(_pdfs(), [plane[..., 0], plane[..., 4]], plane[..., 1:4])
+    padded = torch.zeros(SHAPE[0] + 2, SHAPE[1], SHAPE[2] + 3)
+    assert _own_memory(_pdfs(), [padded[1:-1, :, :SHAPE[2]]], None)
+
+
+@pytest.mark.parametrize("extra", [0, 4])
+def test_the_populations_own_memory_is_shared(extra):
+    pdfs = _pdfs(extra=extra)
+    f = pdfs[..., :19]
+    assert not _own_memory(f, [f[..., 0]], None)
+    assert not _own_memory(f, [], f[..., 5:8])
+    assert not _own_memory(f, [_c(*SHAPE)], f[..., 16:19])
+    if extra:
+        assert _own_memory(f, [pdfs[..., 19]], pdfs[..., 20:23])
+
+
+def test_shared_outputs():
+    rho, u = _c(*SHAPE), _c(*SHAPE, 3)
+    assert not _own_memory(_pdfs(), [rho, rho], u)
+    assert not _own_memory(_pdfs(), [u[..., 1]], u)
+    assert not _own_memory(_pdfs(), [_c(1, *SHAPE[1:]).expand(*SHAPE)], None)
+    base = torch.zeros(200)
+    sliding = base.as_strided(SHAPE, (1, 2, 3))   # elements of one field on top of each other
+    assert not _own_memory(_pdfs(), [sliding], None)
+    assert not _own_memory(_pdfs(), [], base.as_strided(SHAPE + (3,), (1, 6, 30, 6)))
+
+
+@pytest.mark.gpu
+def test_shared_memory_is_staged():
+    from lbmpy_amd import LBMConfig, LBStencil, create_lb_method, compile_macroscopic_values_getter
+    from lbmpy_amd.sweep import create_pdf_array
+    m = create_lb_method(LBMConfig(stencil=LBStencil("D3Q19"), relaxation_rate=1.7, compressible=True))
+    shape = (70, 33, 20)
+    pdf = create_pdf_array(shape, 19, 0, "float32")
+    pdf.copy_(0.01 * torch.randn(pdf.shape, device="cuda"))
+    get = compile_macroscopic_values_getter(m, ["density", "density_deviation", "velocity"], ghost_layers=0)
+    rho, dev = torch.empty(shape, device="cuda"), torch.empty(shape, device="cuda")
+    u = torch.empty(shape + (3,), device="cuda")
+    get(pdf, density=rho, density_deviation=dev, velocity=u)
+    # into the populations themselves, and into one field after the other: the last one written stays
+    own = pdf.clone(memory_format=torch.preserve_format)
+    get(own, density=own[..., 0], density_deviation=own[..., 9], velocity=own[..., 1:4])
+    assert torch.equal(own[..., 0], rho) and torch.equal(own[..., 9], dev) and torch.equal(own[..., 1:4], u)
+    assert torch.equal(own[..., 10:], pdf[..., 10:])
+    v = torch.empty(shape + (3,), device="cuda")
+    get(pdf, density=v[..., 0], density_deviation=v[..., 0], velocity=v)
+    assert torch.equal(v, u)
+    # interleaved components take the direct way, and give the same
+    cell = torch.empty(shape + (5,), device="cuda")
+    get(pdf, density=cell[..., 0], density_deviation=cell[..., 4], velocity=cell[..., 1:4])
+    assert torch.equal(cell[..., 0], rho) and torch.equal(cell[..., 4], dev) and torch.equal(cell[..., 1:4], u)
