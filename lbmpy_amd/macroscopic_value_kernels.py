@@ -205,13 +205,14 @@ def _own_memory(pdfs, scalars, velocity):
 
 
 def _get_in_place(ctx, pdfs, density, velocity, code, density_deviation):
-    """The getter straight into the output tensors; False where they do not admit it (the kernel takes FP64 and FP32
-    fields of any order, shaped like the PDFs)."""
+    """The getter straight into the output tensors; False where they do not admit it (the kernel takes plain FP64 and FP32
+    fields of any order, shaped like the PDFs, that torch would write without further bookkeeping)."""
     D, g = ctx.D, ctx.g
     spatial = tuple(pdfs.shape[:-1])
     scalars = [t for t in (density, density_deviation) if t is not None]
     fields = scalars + ([velocity] if velocity is not None else [])
-    if not all(isinstance(t, torch.Tensor) and t.device == pdfs.device and not t.requires_grad for t in fields) or \
+    if not all(type(t) is torch.Tensor and t.device == pdfs.device and t.layout == torch.strided and not t.requires_grad
+               and not t.is_neg() and not t.is_inference() for t in fields) or \
             len({t.dtype for t in fields}) != 1 or fields[0].dtype not in (torch.float64, torch.float32) or \
             any(tuple(t.shape) != spatial for t in scalars) or len({t.stride() for t in scalars}) > 1 or \
             (velocity is not None and tuple(velocity.shape) != spatial + (D,)) or \
@@ -233,6 +234,7 @@ def _get_in_place(ctx, pdfs, density, velocity, code, density_deviation):
     d = ctx.descriptor(pdfs)
     nat.check(nat.load().lbm355_get_fields(ctypes.byref(d), ctypes.c_void_p(pdfs.data_ptr()), ctypes.byref(o), code,
                                            nat.current_stream_handle()))
+    torch.autograd.graph.increment_version(fields)   # as torch's own writes do, for what autograd saved
     return True
 
 

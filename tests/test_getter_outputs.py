@@ -83,3 +83,30 @@ def test_shared_memory_is_staged():
     cell = torch.empty(shape + (5,), device="cuda")
     get(pdf, density=cell[..., 0], density_deviation=cell[..., 4], velocity=cell[..., 1:4])
     assert torch.equal(cell[..., 0], rho) and torch.equal(cell[..., 4], dev) and torch.equal(cell[..., 1:4], u)
+
+
+@pytest.mark.gpu
+def test_torch_knows_of_the_write():
+    from lbmpy_amd import LBMConfig, LBStencil, create_lb_method, compile_macroscopic_values_getter
+    from lbmpy_amd.sweep import create_pdf_array
+    m = create_lb_method(LBMConfig(stencil=LBStencil("D2Q9"), relaxation_rate=1.7))
+    pdf = create_pdf_array((8, 7), 9, 0, "float64")
+    pdf.fill_(0.01)
+    get = compile_macroscopic_values_getter(m, ["density"], ghost_layers=0)
+    rho = torch.ones(8, 7, dtype=torch.float64, device="cuda")
+    w = torch.ones_like(rho, requires_grad=True)
+    loss = (w * rho).sum()          # saves rho
+    get(pdf, density=rho)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        loss.backward()
+    # views with a pending negation, and tensors made in inference mode
+    neg = torch.view_as_complex(torch.zeros(8, 7, 2, dtype=torch.float64, device="cuda")).conj().imag
+    assert neg.is_neg()
+    get(pdf, density=neg)
+    assert torch.equal(neg, rho)
+    with torch.inference_mode():
+        frozen = torch.ones(8, 7, dtype=torch.float64, device="cuda")
+        get(pdf, density=frozen)
+    assert torch.equal(frozen, rho)
+    with pytest.raises(RuntimeError):
+        get(pdf, density=frozen)
