@@ -191,6 +191,20 @@ struct CellDivider {
   }
 };
 
+// Calls f(y0, ny, z0, nz) for boxes of whole rows that cover nx x ny x nz cells, each of fewer than 2^31 cells; as long
+// as f returns 0.
+template <class F>
+int for_cell_boxes(int nx, int ny, int nz, F f) {
+  const int64_t most = (int64_t(1) << 31) - 1, rows = most / nx;
+  const int by = (int)(ny < rows ? ny : rows), bz = by < ny ? 1 : (int)(nz < rows / ny ? nz : rows / ny);
+  for (int64_t z = 0; z < nz; z += bz)
+    for (int64_t y = 0; y < ny; y += by) {
+      const int rc = f((int)y, (int)(ny - y < by ? ny - y : by), (int)z, (int)(nz - z < bz ? nz - z : bz));
+      if (rc) return rc;
+    }
+  return 0;
+}
+
 // Consecutive workgroups go to the 8 XCDs in turn, each with an L2 of its own.  XcdOrder renumbers them so that runs of
 // `chunk` neighbouring block numbers share an XCD: within every group of 8 chunk blocks, the blocks of one XCD take
 // one run.  The blocks after the last whole group, and all of them with chunk <= 1, keep their numbers.  `backwards`: from

@@ -127,6 +127,8 @@ struct GetArgs {
   int face[3];
   int flags;
   double force[3];
+  int y0, z0;                 // the box of cells of a launch that numbers them (for_cell_boxes)
+  uint32_t cells;
   CellDivider row, plane;
   lbm355_macroscopic_out out;
 };
@@ -187,8 +189,8 @@ template <class S, int PAT, class TS>
 __global__ void __launch_bounds__(256) get_macroscopic_kernel(const TS* pdf, GetArgs a) {
   const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t r = a.row.quotient(t), p = a.plane.quotient(r);
-  const int x = (int)(t - r * a.row.d), y = (int)(r - p * a.plane.d), z = (int)p;
-  if (t >= a.row.d * a.plane.d * (uint32_t)a.nz) return;
+  const int x = (int)(t - r * a.row.d), y = a.y0 + (int)(r - p * a.plane.d), z = a.z0 + (int)p;
+  if (t >= a.cells) return;
   double rho, u[3];
   cell_macroscopic<S, PAT, TS>(pdf, a, x, y, z, rho, u);
   const lbm355_macroscopic_out& o = a.out;
@@ -339,8 +341,7 @@ int set_eq_launch(const lbm355_sweep_desc* d, void* pdf, const double* rho, cons
 
 template <class S, class TS, bool TURNED>
 int get_launch(const GetArgs& a, const void* pdf, int last_pattern, hipStream_t s) {
-  const int64_t cells = (int64_t)a.nx * a.ny * a.nz;
-  dim3 grid((unsigned)((cells + 255) / 256)), block(256);
+  dim3 grid((a.cells + 255) / 256), block(256);
   if (TURNED) grid = dim3((a.nx + 63) / 64, ((S::D == 3 ? a.nz : a.ny) + TURN - 1) / TURN, S::D == 3 ? a.ny : 1);
 #define LBM_GET(P)                                                                                       \
   case P:                                                                                                \
@@ -377,12 +378,20 @@ template <class S, class TS>
 int get_order(const GetArgs& a, const void* pdf, int last, hipStream_t s) {
   const bool x_first = (!(a.out.density || a.out.density_deviation) || a.out.scalar_stride[0] == 1) &&
                        (!a.out.velocity || a.out.vector_stride[0] == 1);
-  return x_first ? get_launch<S, TS, false>(a, pdf, last, s) : get_launch<S, TS, true>(a, pdf, last, s);
+  if (!x_first) return get_launch<S, TS, true>(a, pdf, last, s);
+  return for_cell_boxes(a.nx, a.ny, a.nz, [&](int y, int ny, int z, int nz) {
+    GetArgs box = a;
+    box.y0 = y;
+    box.z0 = z;
+    box.cells = (uint32_t)((int64_t)a.nx * ny * nz);
+    box.plane = CellDivider::of((uint32_t)ny);
+    return get_launch<S, TS, false>(box, pdf, last, s);
+  });
 }
 
 template <class S>
 int get_dtype(const lbm355_sweep_desc* d, const void* pdf, const lbm355_macroscopic_out& out, int last, hipStream_t s) {
-  GetArgs a;
+  GetArgs a = {};
   a.nx = d->nx;
   a.ny = d->ny;
   a.nz = d->nz;
@@ -396,7 +405,6 @@ int get_dtype(const lbm355_sweep_desc* d, const void* pdf, const lbm355_macrosco
   }
   a.flags = d->flags;
   a.row = CellDivider::of((uint32_t)d->nx);
-  a.plane = CellDivider::of((uint32_t)d->ny);
   a.out = out;
   if (d->store_dtype == LBM355_F64) return get_order<S, double>(a, pdf, last, s);
   if (d->store_dtype == LBM355_F32) return get_order<S, float>(a, pdf, last, s);
@@ -461,9 +469,7 @@ int lbm355_get_fields(const lbm355_sweep_desc* d, const void* pdf, const lbm355_
   if (d->store_dtype < 0 || d->store_dtype > 2) return fail2(LBM355_ERR_ARG, "bad dtype");
   if (out->dtype != LBM355_F64 && out->dtype != LBM355_F32) return fail2(LBM355_ERR_ARG, "output fields are F64 or F32");
   if (last_pattern < LBM355_PULL || last_pattern > LBM355_PUSH) return fail2(LBM355_ERR_ARG, "bad pattern");
-  if (d->nx <= 0 || d->ny <= 0 || d->nz <= 0 || d->ny > 65535 || d->nz > 65535 ||
-      (int64_t)d->nx * d->ny * d->nz >= (int64_t(1) << 31))
-    return fail2(LBM355_ERR_ARG, "bad interior size");
+  if (d->nx <= 0 || d->ny <= 0 || d->nz <= 0) return fail2(LBM355_ERR_ARG, "bad interior size");
   if (table_pattern(last_pattern))
     for (int a = 0; a < (d->stencil == LBM355_D2Q9 ? 2 : 3); ++a)
       if (d->face[a] == LBM355_FACE_NOSLIP) return fail2(LBM355_ERR_ARG, "Eso patterns have no fused NoSlip faces");

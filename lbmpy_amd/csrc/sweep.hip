@@ -657,35 +657,36 @@ int boundary_args(const lbm355_boundary_desc* d, const void* pdf, const int32_t*
   return LBM355_OK;
 }
 
-bool cells_below_2_31(const lbm355_sweep_desc* d) {
-  return d->nx > 0 && d->ny > 0 && d->nz > 0 && (int64_t)d->nx * d->ny < (int64_t(1) << 31) &&
-         (int64_t)d->nx * d->ny * d->nz < (int64_t(1) << 31);
-}
+bool has_cells(const lbm355_sweep_desc* d) { return d->nx > 0 && d->ny > 0 && d->nz > 0; }
 
 template <class S, class TS>
 int launch_reduce(const lbm355_sweep_desc* d, const void* pdf, double* out, hipStream_t s) {
   hipLaunchKernelGGL(zero4_kernel, dim3(1), dim3(64), 0, s, out);
-  const uint32_t cells = (uint32_t)((int64_t)d->nx * d->ny * d->nz);
-  const unsigned blocks = (cells + 255) / 256;
-  hipLaunchKernelGGL((reduce_kernel<S, TS>), dim3(blocks < REDUCE_BLOCKS ? blocks : REDUCE_BLOCKS), dim3(256), 0, s,
-                     (const TS*)pdf, CellDivider::of((uint32_t)d->nx), CellDivider::of((uint32_t)d->ny), cells,
-                     d->ghost_layers, d->stride_y, d->stride_z, d->stride_q,
-                     (d->flags & LBM355_FLAG_ZERO_CENTERED) ? 1 : 0, out);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail(LBM355_ERR_LAUNCH, std::string("launch failed: ") + hipGetErrorString(e));
-  return LBM355_OK;
+  return for_cell_boxes(d->nx, d->ny, d->nz, [&](int y, int ny, int z, int nz) {
+    const uint32_t cells = (uint32_t)((int64_t)d->nx * ny * nz);
+    const unsigned blocks = (cells + 255) / 256;
+    hipLaunchKernelGGL((reduce_kernel<S, TS>), dim3(blocks < REDUCE_BLOCKS ? blocks : REDUCE_BLOCKS), dim3(256), 0, s,
+                       (const TS*)pdf + y * d->stride_y + z * d->stride_z, CellDivider::of((uint32_t)d->nx),
+                       CellDivider::of((uint32_t)ny), cells, d->ghost_layers, d->stride_y, d->stride_z, d->stride_q,
+                       (d->flags & LBM355_FLAG_ZERO_CENTERED) ? 1 : 0, out);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(LBM355_ERR_LAUNCH, std::string("launch failed: ") + hipGetErrorString(e));
+    return (int)LBM355_OK;
+  });
 }
 
 template <class S, class TS>
 int launch_nonfinite(const lbm355_sweep_desc* d, const void* pdf, unsigned long long* out, hipStream_t s) {
   hipLaunchKernelGGL(zero1_kernel, dim3(1), dim3(64), 0, s, out);
-  const uint32_t cells = (uint32_t)((int64_t)d->nx * d->ny * d->nz);
-  hipLaunchKernelGGL((nonfinite_kernel<S, TS>), dim3((cells + 255) / 256), dim3(256), 0, s, (const TS*)pdf,
-                     CellDivider::of((uint32_t)d->nx), CellDivider::of((uint32_t)d->ny), cells, d->ghost_layers,
-                     d->stride_y, d->stride_z, d->stride_q, out);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail(LBM355_ERR_LAUNCH, std::string("launch failed: ") + hipGetErrorString(e));
-  return LBM355_OK;
+  return for_cell_boxes(d->nx, d->ny, d->nz, [&](int y, int ny, int z, int nz) {
+    const uint32_t cells = (uint32_t)((int64_t)d->nx * ny * nz);
+    hipLaunchKernelGGL((nonfinite_kernel<S, TS>), dim3((cells + 255) / 256), dim3(256), 0, s,
+                       (const TS*)pdf + y * d->stride_y + z * d->stride_z, CellDivider::of((uint32_t)d->nx),
+                       CellDivider::of((uint32_t)ny), cells, d->ghost_layers, d->stride_y, d->stride_z, d->stride_q, out);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(LBM355_ERR_LAUNCH, std::string("launch failed: ") + hipGetErrorString(e));
+    return (int)LBM355_OK;
+  });
 }
 
 template <class S>
@@ -868,7 +869,7 @@ int lbm355_boundary_groups(const lbm355_boundary_desc* d, int32_t n_groups, void
 
 int lbm355_reduce_conserved(const lbm355_sweep_desc* d, const void* pdf, double* out, void* stream) {
   if (!d || !pdf || !out) return fail(LBM355_ERR_ARG, "NULL argument");
-  if (!cells_below_2_31(d)) return fail(LBM355_ERR_ARG, "bad interior size");
+  if (!has_cells(d)) return fail(LBM355_ERR_ARG, "bad interior size");
   hipStream_t s = (hipStream_t)stream;
   if (d->stencil == LBM355_D2Q9) return reduce_dtype<D2Q9>(d, pdf, out, s);
   if (d->stencil == LBM355_D3Q19) return reduce_dtype<D3Q19>(d, pdf, out, s);
@@ -878,7 +879,7 @@ int lbm355_reduce_conserved(const lbm355_sweep_desc* d, const void* pdf, double*
 
 int lbm355_count_nonfinite(const lbm355_sweep_desc* d, const void* pdf, uint64_t* out, void* stream) {
   if (!d || !pdf || !out) return fail(LBM355_ERR_ARG, "NULL argument");
-  if (!cells_below_2_31(d)) return fail(LBM355_ERR_ARG, "bad interior size");
+  if (!has_cells(d)) return fail(LBM355_ERR_ARG, "bad interior size");
   hipStream_t s = (hipStream_t)stream;
   unsigned long long* o = reinterpret_cast<unsigned long long*>(out);
   if (d->stencil == LBM355_D2Q9) return nonfinite_dtype<D2Q9>(d, pdf, o, s);
