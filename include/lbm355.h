@@ -163,6 +163,22 @@ typedef struct lbm355_sweep_desc {
 int lbm355_sweep(const lbm355_sweep_desc* desc, const void* pdf_src, void* pdf_dst, void* density_out,
                  void* velocity_out, void* stream);
 
+/* How a sweep covers the cells and reaches memory.  lbm355_sweep chooses by the populations' size and alignment; results
+ * do not depend on it. */
+#define LBM355_ACCESS_ROWS 0   /* one block per whole periodic row (nx a multiple of 64), non-temporal accesses */
+#define LBM355_ACCESS_WAVES 1  /* rows of whole wavefronts, non-temporal accesses at the cell itself */
+#define LBM355_ACCESS_LINES 2  /* consecutive cells, non-temporal accesses at the cell itself */
+#define LBM355_ACCESS_CACHED 3 /* consecutive cells, regular accesses, for populations that the caches hold */
+#define LBM355_ACCESS_SHARED 4 /* consecutive cells, regular accesses, every other sweep backwards */
+
+/* The mode that lbm355_sweep takes for these arguments (the arrays' addresses count, they are not read), or the
+ * negative of an error code. */
+int32_t lbm355_sweep_access(const lbm355_sweep_desc* desc, const void* pdf_src, const void* pdf_dst);
+
+/* lbm355_sweep in a given mode, LBM355_ERR_UNSUPPORTED where the pattern has no such kernel for this domain. */
+int lbm355_sweep_with_access(const lbm355_sweep_desc* desc, const void* pdf_src, void* pdf_dst, void* density_out,
+                             void* velocity_out, int32_t access, void* stream);
+
 /* Number of compute_dtype elements the method table of (stencil, family) holds. */
 int64_t lbm355_table_elements(int32_t stencil, int32_t family);
 

@@ -63,8 +63,10 @@ class MacroscopicOut(ctypes.Structure):
                 ("scalar_stride", c_int64 * 3), ("vector_stride", c_int64 * 4), ("dtype", c_int32), ("pad", c_int32)]
 
 
-EXPORTED = ("lbm355_sweep", "lbm355_table_elements", "lbm355_noslip_links", "lbm355_reduce_conserved",
-            "lbm355_count_nonfinite",
+ACCESS_ROWS, ACCESS_WAVES, ACCESS_LINES, ACCESS_CACHED, ACCESS_SHARED = 0, 1, 2, 3, 4
+
+EXPORTED = ("lbm355_sweep", "lbm355_sweep_access", "lbm355_sweep_with_access", "lbm355_table_elements",
+            "lbm355_noslip_links", "lbm355_reduce_conserved", "lbm355_count_nonfinite",
             "lbm355_set_equilibrium", "lbm355_get_macroscopic", "lbm355_get_fields", "lbm355_stream_copy", "lbm355_desc_size",
             "lbm355_last_error", "lbm355_version", "lbm355_batch_create", "lbm355_batch_sweep",
             "lbm355_batch_info", "lbm355_batch_destroy", "lbm355_batch_sweep_static", "lbm355_closure_params_size",
@@ -90,6 +92,11 @@ def load(path=None):
     lib = ctypes.CDLL(path, mode=ctypes.RTLD_GLOBAL)
     lib.lbm355_sweep.argtypes = [ctypes.POINTER(SweepDesc), c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]
     lib.lbm355_sweep.restype = c_int32
+    lib.lbm355_sweep_access.argtypes = [ctypes.POINTER(SweepDesc), c_void_p, c_void_p]
+    lib.lbm355_sweep_access.restype = c_int32
+    lib.lbm355_sweep_with_access.argtypes = [ctypes.POINTER(SweepDesc), c_void_p, c_void_p, c_void_p, c_void_p, c_int32,
+                                             c_void_p]
+    lib.lbm355_sweep_with_access.restype = c_int32
     lib.lbm355_table_elements.argtypes = [c_int32, c_int32]
     lib.lbm355_table_elements.restype = c_int64
     lib.lbm355_noslip_links.argtypes = [c_int32, c_int32, c_int32, c_void_p, c_int64, c_int64, c_int64, c_void_p,

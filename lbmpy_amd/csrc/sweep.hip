@@ -480,13 +480,20 @@ int validate(const lbm355_sweep_desc* d) {
   return LBM355_OK;
 }
 
-template <class TC>
-int launch_sweep(const lbm355_sweep_desc* d, const void* src, void* dst, void* rho, void* u, hipStream_t s) {
-  if (table_pattern(d->pattern)) return lbm355_launch_sweep_eso(d, src, dst, rho, u, s);
-  const bool walls = has_walls(d);
-  size_t lds = 0;
+// AA odd streams its populations only by rows: it reaches none but the centre's at the cell itself.
+StreamedModes streamed_modes(const lbm355_sweep_desc* d, size_t* row_lds) {
+  const bool waves = d->nx % 64 == 0;
+  if (table_pattern(d->pattern)) return {lbm355_eso_row_lds(d, row_lds), waves, false};
   const bool odd = d->pattern == LBM355_AA_ODD;
-  const SweepLaunch l = sweep_launch(d, src, dst, use_rowlds(d, &lds), !odd, !odd);
+  return {use_rowlds(d, row_lds), waves && !odd, !odd};
+}
+
+template <class TC>
+int launch_sweep(const lbm355_sweep_desc* d, const void* src, void* dst, void* rho, void* u, int access, size_t lds,
+                 hipStream_t s) {
+  const SweepLaunch l = sweep_launch(d, src, dst, (AccessMode)access);
+  if (table_pattern(d->pattern)) return lbm355_launch_sweep_eso(d, src, dst, rho, u, l, lds, s);
+  const bool walls = has_walls(d);
   void* k = pick_kernel<TC>(d, walls, l.mode);
   if (!k) return fail(LBM355_ERR_UNSUPPORTED, "no kernel for this stencil/family/dtype combination");
   SweepArgs<TC> a = make_args<TC>(d, src, dst, rho, u);
@@ -704,14 +711,9 @@ int reduce_dtype(const lbm355_sweep_desc* d, const void* pdf, double* out, hipSt
   if (d->store_dtype == LBM355_F16) return launch_reduce<S, _Float16>(d, pdf, out, s);
   return fail(LBM355_ERR_ARG, "bad dtype");
 }
-}  // namespace
-
-int lbm355_validate_desc(const lbm355_sweep_desc* d) { return validate(d); }
-
-extern "C" {
-
-int lbm355_sweep(const lbm355_sweep_desc* d, const void* pdf_src, void* pdf_dst, void* density_out,
-                 void* velocity_out, void* stream) {
+// What a sweep refuses.
+int check_sweep(const lbm355_sweep_desc* d, const void* pdf_src, const void* pdf_dst, const void* density_out,
+                const void* velocity_out) {
   int rc = validate(d);
   if (rc) return rc;
   if (!pdf_src || !pdf_dst) return fail(LBM355_ERR_ARG, "PDF pointers must not be NULL");
@@ -775,9 +777,43 @@ int lbm355_sweep(const lbm355_sweep_desc* d, const void* pdf_src, void* pdf_dst,
     if ((velocity_out || d->velocity_in) && d->out_stride_c < volume)
       return fail(LBM355_ERR_ARG, "out_stride_c smaller than one component");
   }
-  hipStream_t s = (hipStream_t)stream;
-  if (d->compute_dtype == LBM355_F64) return launch_sweep<double>(d, pdf_src, pdf_dst, density_out, velocity_out, s);
-  return launch_sweep<float>(d, pdf_src, pdf_dst, density_out, velocity_out, s);
+  return LBM355_OK;
+}
+
+// access: an ACCESS mode, or -1 for the one that choose_access takes
+int sweep(const lbm355_sweep_desc* d, const void* src, void* dst, void* rho, void* u, int access, void* stream) {
+  const int rc = check_sweep(d, src, dst, rho, u);
+  if (rc) return rc;
+  size_t lds = 0;
+  const StreamedModes modes = streamed_modes(d, &lds);
+  if (access == -1) access = choose_access(d, src, dst, modes);
+  if (!admits(modes, access)) return fail(LBM355_ERR_UNSUPPORTED, "this sweep has no kernel of that access mode");
+  if (d->compute_dtype == LBM355_F64)
+    return launch_sweep<double>(d, src, dst, rho, u, access, lds, (hipStream_t)stream);
+  return launch_sweep<float>(d, src, dst, rho, u, access, lds, (hipStream_t)stream);
+}
+}  // namespace
+
+int lbm355_validate_desc(const lbm355_sweep_desc* d) { return validate(d); }
+
+extern "C" {
+
+int lbm355_sweep(const lbm355_sweep_desc* d, const void* pdf_src, void* pdf_dst, void* density_out,
+                 void* velocity_out, void* stream) {
+  return sweep(d, pdf_src, pdf_dst, density_out, velocity_out, -1, stream);
+}
+
+int lbm355_sweep_with_access(const lbm355_sweep_desc* d, const void* pdf_src, void* pdf_dst, void* density_out,
+                             void* velocity_out, int32_t access, void* stream) {
+  if (access < 0) return fail(LBM355_ERR_ARG, "unknown access mode");
+  return sweep(d, pdf_src, pdf_dst, density_out, velocity_out, access, stream);
+}
+
+int32_t lbm355_sweep_access(const lbm355_sweep_desc* d, const void* pdf_src, const void* pdf_dst) {
+  const int rc = check_sweep(d, pdf_src, pdf_dst, nullptr, nullptr);
+  if (rc) return -rc;
+  size_t lds = 0;
+  return choose_access(d, pdf_src, pdf_dst, streamed_modes(d, &lds));
 }
 
 int64_t lbm355_table_elements(int32_t stencil, int32_t family) {
@@ -890,7 +926,7 @@ int lbm355_count_nonfinite(const lbm355_sweep_desc* d, const void* pdf, uint64_t
 
 const char* lbm355_last_error(void) { return g_err.c_str(); }
 
-int32_t lbm355_version(void) { return 9; }
+int32_t lbm355_version(void) { return 10; }
 
 #ifndef LBM355_SOURCE_HASH
 #define LBM355_SOURCE_HASH "unknown"

@@ -347,8 +347,12 @@ __device__ __forceinline__ void sweep_cell(const SweepArgs<TC>& a, int x, int y,
 // ACCESS_ROWS    one block per whole periodic row, x-shifts through LDS, non-temporal accesses (the row kernels);
 // ACCESS_WAVES   one thread per cell, rows of whole wavefronts, accesses at the cell itself non-temporal;
 // ACCESS_LINES   the same with rows of any length, consecutive in memory;
-// ACCESS_CACHED  one thread per cell, regular accesses.
-enum AccessMode { ACCESS_ROWS, ACCESS_WAVES, ACCESS_LINES, ACCESS_CACHED };
+// ACCESS_CACHED  one thread per cell, regular accesses, one run of blocks per XCD;
+// ACCESS_SHARED  the same kernel with short runs, which every other sweep goes backwards.
+enum AccessMode {
+  ACCESS_ROWS = LBM355_ACCESS_ROWS, ACCESS_WAVES = LBM355_ACCESS_WAVES, ACCESS_LINES = LBM355_ACCESS_LINES,
+  ACCESS_CACHED = LBM355_ACCESS_CACHED, ACCESS_SHARED = LBM355_ACCESS_SHARED
+};
 
 // The cell of this thread, or false beyond the last cell.  Threads number the cells consecutively over rows and
 // planes, so that wavefronts are full whatever nx is; with ACCESS_WAVES, blocks take up to 256 cells of one row, and y
@@ -442,6 +446,33 @@ inline bool has_walls(const lbm355_sweep_desc* d) {
   return false;
 }
 
+// The streamed modes that a sweep has a kernel for.
+struct StreamedModes {
+  bool rows, waves, lines;
+};
+
+inline bool admits(const StreamedModes& m, int access) {
+  switch (access) {
+    case ACCESS_ROWS: return m.rows;
+    case ACCESS_WAVES: return m.waves;
+    case ACCESS_LINES: return m.lines;
+    case ACCESS_CACHED: case ACCESS_SHARED: return true;
+  }
+  return false;
+}
+
+inline AccessMode choose_access(const lbm355_sweep_desc* d, const void* src, const void* dst, const StreamedModes& m) {
+  const bool in_place = src == dst;
+  const int64_t bytes = population_bytes(d, in_place);
+  if (fits_cache(bytes, d->store_dtype, in_place)) return ACCESS_CACHED;
+  if (!cached_anyway(bytes, d->store_dtype, in_place, has_walls(d)) && starts_lines(d, src, dst)) {
+    if (m.rows) return ACCESS_ROWS;
+    if (m.waves) return ACCESS_WAVES;
+    if (m.lines) return ACCESS_LINES;
+  }
+  return ACCESS_SHARED;
+}
+
 struct SweepLaunch {
   AccessMode mode;
   dim3 grid, block;
@@ -449,25 +480,21 @@ struct SweepLaunch {
   bool half_cache;   // the populations take at most HALF_CACHE_BYTES
 };
 
-// row_kernel, waves_kernel, lines_kernel: whether the caller has a kernel of that mode for this sweep.
-inline SweepLaunch sweep_launch(const lbm355_sweep_desc* d, const void* src, const void* dst, bool row_kernel,
-                                bool waves_kernel, bool lines_kernel) {
+inline SweepLaunch sweep_launch(const lbm355_sweep_desc* d, const void* src, const void* dst, AccessMode access) {
   const bool in_place = src == dst;
   const int64_t bytes = population_bytes(d, in_place);
-  const bool fits = fits_cache(bytes, d->store_dtype, in_place), half = bytes <= HALF_CACHE_BYTES;
-  const bool lines = !fits && !cached_anyway(bytes, d->store_dtype, in_place, has_walls(d)) && starts_lines(d, src, dst);
-  if (row_kernel && lines) return {ACCESS_ROWS, dim3(1, d->ny, d->nz), dim3(d->nx), XcdOrder::of(1, 1), half};
-  if (waves_kernel && lines && d->nx % 64 == 0) {
+  const bool half = bytes <= HALF_CACHE_BYTES;
+  if (access == ACCESS_ROWS) return {access, dim3(1, d->ny, d->nz), dim3(d->nx), XcdOrder::of(1, 1), half};
+  if (access == ACCESS_WAVES) {
     const unsigned bx = d->nx < 256 ? d->nx : 256;
-    return {ACCESS_WAVES, dim3((d->nx + bx - 1) / bx, d->ny, d->nz), dim3(bx), XcdOrder::of(1, 1), half};
+    return {access, dim3((d->nx + bx - 1) / bx, d->ny, d->nz), dim3(bx), XcdOrder::of(1, 1), half};
   }
   const int64_t cells = (int64_t)d->nx * d->ny * d->nz;
   const unsigned bx = cells < SMALL_CELLS ? 64 : 256;
   const unsigned blocks = (unsigned)((cells + bx - 1) / bx);
-  if (lines_kernel && lines) return {ACCESS_LINES, dim3(blocks), dim3(bx), XcdOrder::of(blocks, 1), half};
-  const bool backwards = !fits && meets_cached(bytes, in_place) && backwards_sweep(d->pattern, src, dst);
-  const unsigned chunk = fits ? blocks / 8 : SHARED_LINES_CHUNK;
-  return {ACCESS_CACHED, dim3(blocks), dim3(bx), XcdOrder::of(blocks, chunk, backwards), half};
+  const unsigned chunk = access == ACCESS_LINES ? 1 : access == ACCESS_CACHED ? blocks / 8 : SHARED_LINES_CHUNK;
+  const bool backwards = access == ACCESS_SHARED && meets_cached(bytes, in_place) && backwards_sweep(d->pattern, src, dst);
+  return {access, dim3(blocks), dim3(bx), XcdOrder::of(blocks, chunk, backwards), half};
 }
 
 // Kernel arguments from a public descriptor (include/lbm355.h).
@@ -518,4 +545,6 @@ int lbm355_validate_desc(const lbm355_sweep_desc* d);
 
 // sweeps of the Eso patterns and push (sweep_eso.hip); the descriptor has been validated
 int lbm355_launch_sweep_eso(const lbm355_sweep_desc* d, const void* src, void* dst, void* rho, void* u,
-                            hipStream_t s);
+                            const lbm355::SweepLaunch& l, size_t row_lds, hipStream_t s);
+// whether they have a row kernel for this domain, and the LDS bytes of a row
+bool lbm355_eso_row_lds(const lbm355_sweep_desc* d, size_t* lds_bytes);

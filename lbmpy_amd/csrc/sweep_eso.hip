@@ -39,16 +39,17 @@ void* eso_pick(const lbm355_sweep_desc* d, int mode) {
 
 using namespace lbm355;
 
-int lbm355_launch_sweep_eso(const lbm355_sweep_desc* d, const void* src, void* dst, void* rho, void* u,
-                            hipStream_t s) {
+bool lbm355_eso_row_lds(const lbm355_sweep_desc* d, size_t* lds_bytes) {
   // whole periodic rows of at most 512 cells (whole wavefronts) go through the row-staged kernel
   const size_t es = d->store_dtype == LBM355_F64 ? 8 : (d->store_dtype == LBM355_F32 ? 4 : 2);
   const int rows_needed = d->stencil == LBM355_D2Q9 ? eso_max_rows<D2Q9>()
                           : d->stencil == LBM355_D3Q19 ? eso_max_rows<D3Q19>() : eso_max_rows<D3Q27>();
-  const size_t lds = (size_t)rows_needed * d->nx * es;
-  const bool row_kernel = d->face[0] == LBM355_FACE_PERIODIC && d->nx % 64 == 0 && d->nx <= 512 && lds <= 65536;
-  // the rows that a cell reaches beside its own start on lines, too, only if rows are whole wavefronts
-  const SweepLaunch l = sweep_launch(d, src, dst, row_kernel, true, false);
+  *lds_bytes = (size_t)rows_needed * d->nx * es;
+  return d->face[0] == LBM355_FACE_PERIODIC && d->nx % 64 == 0 && d->nx <= 512 && *lds_bytes <= 65536;
+}
+
+int lbm355_launch_sweep_eso(const lbm355_sweep_desc* d, const void* src, void* dst, void* rho, void* u,
+                            const SweepLaunch& l, size_t lds, hipStream_t s) {
   const bool rows = l.mode == ACCESS_ROWS;
   void* k = d->compute_dtype == LBM355_F64 ? eso_pick<double>(d, l.mode) : eso_pick<float>(d, l.mode);
   if (!k) return lbm355_set_error(LBM355_ERR_UNSUPPORTED, "no Eso kernel for this stencil/family/dtype combination");
