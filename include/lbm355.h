@@ -163,8 +163,8 @@ typedef struct lbm355_sweep_desc {
 int lbm355_sweep(const lbm355_sweep_desc* desc, const void* pdf_src, void* pdf_dst, void* density_out,
                  void* velocity_out, void* stream);
 
-/* How a sweep covers the cells and reaches memory.  lbm355_sweep chooses by the populations' size and alignment; results
- * do not depend on it. */
+/* How a sweep covers the cells and reaches memory.  lbm355_sweep chooses by the populations' size and alignment; the
+ * modes share their arithmetic (the row kernels up to the contraction of products and sums). */
 #define LBM355_ACCESS_ROWS 0   /* one block per whole periodic row (nx a multiple of 64), non-temporal accesses */
 #define LBM355_ACCESS_WAVES 1  /* rows of whole wavefronts, non-temporal accesses at the cell itself */
 #define LBM355_ACCESS_LINES 2  /* consecutive cells, non-temporal accesses at the cell itself */

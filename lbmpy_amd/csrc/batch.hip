@@ -8,7 +8,8 @@
 // covers any ensemble and every wave reaches the end of its loop.  A wave reads its tile's member from
 // a tile -> member map (one wave-uniform load), decodes (x, y, z) with 32-bit arithmetic (a member
 // holds < 2^31 cells) and runs sweep_cell, the same per-cell function as the single-domain sweep
-// (sweep_cell.h): a member's cells get bit-identical results to a single-domain run of that member.
+// (sweep_cell.h): a member's cells get bit-identical results to a single-domain run of that member with one
+// thread per cell (the row kernels may contract a sum otherwise, an ulp).
 //
 // XCD-aware order: MI355X dispatches consecutive workgroups round-robin over its 8 XCDs (each with its
 // own L2).  With `xcd_order`, and for an ensemble that fits the Infinity Cache, the workgroups of one XCD
