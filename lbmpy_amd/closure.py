@@ -11,8 +11,8 @@ calibrated a posteriori on the training flow.  It stands where lbmpy's Smagorins
 Everything runs on the GPU through the C ABI (``include/lbm355.h``):
   * inference fused into the cumulant sweep (``SweepKernel.set_closure``), BF16 MFMA per wavefront;
   * ``lbm355_closure_features`` / ``lbm355_closure_forward`` for batches of samples;
-  * training: ``lbm355_closure_train_step`` (forward, backward and weight gradients on BF16 MFMA with
-    FP32 accumulation) and ``lbm355_closure_adam``.
+  * training: ``lbm355_closure_train_epoch`` (per minibatch forward, backward and weight gradients on BF16 MFMA with
+    FP32 accumulation, and Adam), or its steps ``lbm355_closure_gradient`` and ``lbm355_closure_adam``.
 
 Training data come from the method itself: a fine D3Q27 cumulant run, box-filtered onto the coarse
 grid (:func:`subgrid_samples`).  Torch is used for device memory and for the data plumbing around the
@@ -134,16 +134,21 @@ class ClosureModel:
         return self.nu_scale * torch.nn.functional.softplus(self.forward(features))
 
     def gradient(self, features, targets, blocks=1024):
-        """(loss, grad) of L = mean((softplus(o) - y)^2) at the current parameters (GPU kernels).  `blocks` has no
-        effect: the sums' order is fixed."""
+        """(loss, grad) of L = mean((softplus(o) - y)^2) at the current parameters (GPU kernels).  `blocks` below the
+        default bounds the wavefronts that work on it, whose sums then come in no fixed order."""
         x = features.float().contiguous()
         y = targets.float().contiguous()
         grad = torch.empty(MASTER_SIZE, dtype=torch.float32, device=self.device)
         loss = torch.empty(1, dtype=torch.float32, device=self.device)
         if blocks <= 0:
             raise nat.LbmError("closure gradient: blocks must be positive")
-        nat.check(self.lib.lbm355_closure_gradient(_ptr(self.params), _ptr(x), _ptr(y), x.shape[0], _ptr(grad),
-                                                   _ptr(loss), _ptr(self._workspace()), nat.current_stream_handle()))
+        if blocks < 1024:
+            nat.check(self.lib.lbm355_closure_train_step(_ptr(self.params), _ptr(x), _ptr(y), x.shape[0], _ptr(grad),
+                                                         _ptr(loss), blocks, nat.current_stream_handle()))
+        else:
+            nat.check(self.lib.lbm355_closure_gradient(_ptr(self.params), _ptr(x), _ptr(y), x.shape[0], _ptr(grad),
+                                                       _ptr(loss), _ptr(self._workspace()),
+                                                       nat.current_stream_handle()))
         return loss, grad
 
     def _workspace(self):
