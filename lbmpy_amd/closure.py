@@ -162,28 +162,46 @@ class ClosureModel:
     def train(self, features, targets, epochs=4, batch=65536, lr=2e-3, seed=0, log=None):
         """Adam on minibatches of (features, targets = nu_t / nu_scale); returns the per-epoch mean loss."""
         n = features.shape[0]
-        x = features.float().contiguous()
-        y = targets.float().contiguous()
-        if not (x.is_cuda and y.is_cuda) or x.numel() != n * IN or y.numel() < n:
+        if not (features.is_cuda and targets.is_cuda) or features.numel() != n * IN or targets.dim() < 1 or \
+                targets.shape[0] < n or targets.numel() < n:
             raise ValueError(f"training takes GPU tensors of features ({n}, {IN}) and {n} targets, not "
-                             f"{tuple(x.shape)} on {x.device} and {tuple(y.shape)} on {y.device}")
-        workspace = self._workspace()
-        losses = torch.empty(len(range(0, n, batch)), dtype=torch.float32, device=self.device)
-        nb = len(losses)
+                             f"{tuple(features.shape)} on {features.device} and {tuple(targets.shape)} on "
+                             f"{targets.device}")
+        own = getattr(self.gradient, "__func__", None) is ClosureModel.gradient and \
+            getattr(self.adam_step, "__func__", None) is ClosureModel.adam_step
+        epoch = self._epoch if own else self._epoch_by_steps
+        if own:
+            features, targets = features.float().contiguous(), targets.float().contiguous()
         g = torch.Generator(device=self.device).manual_seed(seed)
         history = []
         for ep in range(epochs):
             perm = torch.randperm(n, generator=g, device=self.device)
-            if nb:
-                nat.check(self.lib.lbm355_closure_train_epoch(
-                    _ptr(self.params), _ptr(self.master), _ptr(self.m), _ptr(self.v), _ptr(x), _ptr(y), _ptr(perm), n,
-                    batch, lr, 0.9, 0.999, 1e-8, self.step, _ptr(losses), _ptr(workspace),
-                    nat.current_stream_handle()))
-                self.step += nb
-            history.append(float(losses.double().sum() / nb))
+            losses = epoch(features, targets, perm, batch, lr)
+            history.append(float(losses.double().sum() / len(losses)))
             if log:
                 log(f"closure training epoch {ep}: loss {history[-1]:.4e}")
         return history
+
+    def _epoch(self, features, targets, perm, batch, lr):
+        n = len(perm)
+        losses = torch.empty(len(range(0, n, batch)), dtype=torch.float32, device=self.device)
+        if len(losses):
+            nat.check(self.lib.lbm355_closure_train_epoch(
+                _ptr(self.params), _ptr(self.master), _ptr(self.m), _ptr(self.v), _ptr(features), _ptr(targets),
+                _ptr(perm), n, batch, lr, 0.9, 0.999, 1e-8, self.step, _ptr(losses), _ptr(self._workspace()),
+                nat.current_stream_handle()))
+            self.step += len(losses)
+        return losses
+
+    def _epoch_by_steps(self, features, targets, perm, batch, lr):
+        """The same through gradient and adam_step, for models that have their own."""
+        losses = []
+        for s in range(0, len(perm), batch):
+            idx = perm[s:s + batch]
+            loss, grad = self.gradient(features[idx], targets[idx])
+            self.adam_step(grad, lr=lr)
+            losses.append(loss[0])
+        return torch.stack(losses) if losses else torch.empty(0)
 
 
 # ---------------------------------------------------------------------- flow fields and diagnostics

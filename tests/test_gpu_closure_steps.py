@@ -50,3 +50,42 @@ def test_gradient_against_the_oracle(n, blocks):
     for a, b in ((co.OFF_W1T, co.OFF_W2T), (co.OFF_W2T, co.OFF_W3), (co.OFF_W3, co.OFF_B1), (co.OFF_B1, co.OFF_B2),
                  (co.OFF_B2, co.OFF_B3), (co.OFF_B3, co.MASTER_SIZE)):
         assert np.linalg.norm(g[a:b] - go[a:b]) <= 3e-2 * np.linalg.norm(go[a:b])
+
+
+def test_training_goes_through_a_models_own_steps():
+    from lbmpy_amd.closure import ClosureModel
+    seen = []
+
+    class Clipped(ClosureModel):
+        def gradient(self, features, targets, blocks=1024):
+            loss, grad = super().gradient(features, targets, blocks)
+            seen.append(len(features))
+            return loss, grad * 0.5
+
+    class Scheduled(ClosureModel):
+        def adam_step(self, grad, lr=1e-3, **kw):
+            super().adam_step(grad, lr=0.0, **kw)
+
+    _, x, y = _setup(1000)
+    plain, clipped, scheduled = (c(seed=3, nu_scale=2e-3) for c in (ClosureModel, Clipped, Scheduled))
+    start = scheduled.master.clone()
+    for m in (plain, clipped, scheduled):
+        assert len(m.train(x, y, epochs=2, batch=300, lr=1e-2)) == 2
+        assert m.step == 8
+    assert seen == [300, 300, 300, 100] * 2
+    assert torch.equal(scheduled.master, start)
+    # a gradient of half the size moves Adam's first moment by half, its second by a quarter
+    by_hand = ClosureModel(seed=3, nu_scale=2e-3)
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    for _ in range(2):
+        perm = torch.randperm(1000, generator=gen, device="cuda")
+        for s in range(0, 1000, 300):
+            _, grad = by_hand.gradient(x[perm[s:s + 300]], y[perm[s:s + 300]])
+            by_hand.adam_step(grad * 0.5, lr=1e-2)
+    assert torch.equal(clipped.master, by_hand.master) and not torch.equal(clipped.master, plain.master)
+
+
+def test_targets_for_every_sample():
+    m, x, _ = _setup(64)
+    with pytest.raises(ValueError):
+        m.train(x, torch.zeros(32, 2, device="cuda"))
