@@ -159,6 +159,8 @@ class ClosureModel:
         nat.check(self.lib.lbm355_closure_adam(_ptr(self.master), _ptr(grad), _ptr(self.m), _ptr(self.v), lr, beta1,
                                                beta2, eps, self.step, _ptr(self.params), nat.current_stream_handle()))
 
+    MOST_CONVERTED = 1 << 30
+
     def train(self, features, targets, epochs=4, batch=65536, lr=2e-3, seed=0, log=None):
         """Adam on minibatches of (features, targets = nu_t / nu_scale); returns the per-epoch mean loss."""
         n = features.shape[0]
@@ -169,9 +171,12 @@ class ClosureModel:
                              f"{targets.device}")
         own = getattr(self.gradient, "__func__", None) is ClosureModel.gradient and \
             getattr(self.adam_step, "__func__", None) is ClosureModel.adam_step
-        epoch = self._epoch if own else self._epoch_by_steps
-        if own:
+        # samples of another type or order are converted at once, up to MOST_CONVERTED bytes, else by minibatches
+        converted = sum(4 * t.numel() for t in (features, targets) if t.dtype != torch.float32 or not t.is_contiguous())
+        whole = own and converted <= self.MOST_CONVERTED
+        if whole:
             features, targets = features.float().contiguous(), targets.float().contiguous()
+        epoch = self._epoch if whole else self._epoch_by_steps
         g = torch.Generator(device=self.device).manual_seed(seed)
         history = []
         for ep in range(epochs):
@@ -194,7 +199,7 @@ class ClosureModel:
         return losses
 
     def _epoch_by_steps(self, features, targets, perm, batch, lr):
-        """The same through gradient and adam_step, for models that have their own."""
+        """The same through gradient and adam_step, which take a minibatch each."""
         losses = []
         for s in range(0, len(perm), batch):
             idx = perm[s:s + batch]

@@ -89,3 +89,24 @@ def test_targets_for_every_sample():
     m, x, _ = _setup(64)
     with pytest.raises(ValueError):
         m.train(x, torch.zeros(32, 2, device="cuda"))
+
+
+@pytest.mark.parametrize("form", ["float64", "columns", "float16 targets"])
+def test_training_converts_no_more_than_its_bound(form):
+    """Samples that need a copy, and more of them than the bound, are converted by minibatches, with the same result."""
+    from lbmpy_amd.closure import ClosureModel
+    n = 200000
+    _, x, y = _setup(n)
+    y = y.half().float()
+    xs, ys = (x.double(), y) if form == "float64" else (x.t().contiguous().t(), y) if form == "columns" else (x, y.half())
+    plain, whole, bounded = (ClosureModel(seed=3, nu_scale=2e-3) for _ in range(3))
+    for m in (whole, bounded):
+        m.lib = _Recorder(m.lib)
+    bounded.MOST_CONVERTED = 4 * ys.numel() - 1
+    plain.train(x, y, epochs=1, batch=30000)
+    for m in (whole, bounded):
+        m.train(xs, ys, epochs=1, batch=30000)
+        assert torch.equal(plain.master, m.master) and plain.step == m.step
+    assert [c[0] for c in whole.lib.calls if "workspace" not in c[0]] == ["lbm355_closure_train_epoch"]
+    sizes = [c[1][3] for c in bounded.lib.calls if c[0] == "lbm355_closure_gradient"]
+    assert sizes == [30000] * 6 + [20000] and not any("epoch" in c[0] for c in bounded.lib.calls)
