@@ -237,6 +237,11 @@ typedef struct lbm355_macroscopic_out {
 int lbm355_get_fields(const lbm355_sweep_desc* desc, const void* pdf, const lbm355_macroscopic_out* out,
                       int32_t last_pattern, void* stream);
 
+/* Pinned host memory, of exactly `bytes` and given back by the free (which first waits for the GPU); NULL if there is
+ * none to be had.  The free returns an error for a pointer that is not of the allocation's. */
+void* lbm355_host_alloc(int64_t bytes);
+int lbm355_host_free(void* memory);
+
 /* Strain-rate tensor S_ab = -1.5 (omega_shear / rho_ref) sum_i c_ia c_ib (f_i - f_eq,i(rho, u)) of the populations
  * the kernel `last_pattern` wrote (read as lbm355_get_macroscopic reads them; rho and the equilibrium velocity u
  * as the collision computes them, rho_ref = rho if compressible, else 1): lbmpy's strain_rate_tensor_getter

@@ -5,9 +5,12 @@ resolves to the HIP runtime torch already loaded: PDF tensors, streams and the
 kernels then live in one runtime.  There is no fallback: if the library is
 missing the import raises.
 """
+import collections
 import ctypes
 import os
+import weakref
 
+import numpy as np
 import torch  # noqa: F401  (must precede the library load, see module docstring)
 
 from .csrc.build import library_path, source_hash
@@ -74,7 +77,8 @@ EXPORTED = ("lbm355_sweep", "lbm355_sweep_access", "lbm355_sweep_with_access", "
             "lbm355_closure_train_step", "lbm355_closure_adam", "lbm355_closure_workspace_floats",
             "lbm355_closure_gradient", "lbm355_closure_train_epoch", "lbm355_boundary_links", "lbm355_boundary_groups",
             "lbm355_copy_boxes",
-            "lbm355_pattern_access", "lbm355_get_strain_rate", "lbm355_plane_copy", "lbm355_valu_probe",
+            "lbm355_pattern_access", "lbm355_get_strain_rate", "lbm355_host_alloc", "lbm355_host_free",
+            "lbm355_plane_copy", "lbm355_valu_probe",
             "lbm355_source_hash")
 
 _lib = None
@@ -113,6 +117,10 @@ def load(path=None):
     lib.lbm355_get_fields.argtypes = [ctypes.POINTER(SweepDesc), c_void_p, ctypes.POINTER(MacroscopicOut), c_int32,
                                       c_void_p]
     lib.lbm355_get_fields.restype = c_int32
+    lib.lbm355_host_alloc.argtypes = [c_int64]
+    lib.lbm355_host_alloc.restype = c_void_p
+    lib.lbm355_host_free.argtypes = [c_void_p]
+    lib.lbm355_host_free.restype = c_int32
     lib.lbm355_stream_copy.argtypes = [c_void_p, c_void_p, c_int64, c_int32, c_void_p]
     lib.lbm355_stream_copy.restype = c_int32
     lib.lbm355_plane_copy.argtypes = [c_int32, c_int32, c_void_p, c_void_p, c_int64, c_int64, c_int32, c_int32,
@@ -199,3 +207,31 @@ def check(rc):
 
 def current_stream_handle():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+
+_freed_later = collections.deque()
+
+
+def _free_pinned(lib, address):
+    """Gives pinned memory back, or notes it for the next call where this thread's stream is being captured (the free
+    waits for the GPU)."""
+    _freed_later.append(address)
+    if not torch.cuda.is_current_stream_capturing():
+        while _freed_later:
+            try:
+                lib.lbm355_host_free(_freed_later.popleft())
+            except IndexError:              # another thread was faster
+                return
+
+
+def pinned_array(shape):
+    """An FP64 numpy array in pinned host memory of exactly its size, which is given back when the array and all its
+    views are gone; None where there is none to be had."""
+    lib = load()
+    nbytes = 8 * int(np.prod(shape, dtype=np.int64))
+    address = lib.lbm355_host_alloc(nbytes)
+    if not address:
+        return None
+    memory = (ctypes.c_char * nbytes).from_address(address)
+    weakref.finalize(memory, _free_pinned, lib, address).atexit = False
+    return np.frombuffer(memory, dtype=np.float64).reshape(shape)

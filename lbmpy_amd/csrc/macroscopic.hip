@@ -411,6 +411,14 @@ int get_dtype(const lbm355_sweep_desc* d, const void* pdf, const lbm355_macrosco
   return get_order<S, _Float16>(a, pdf, last, s);
 }
 
+// Lets this thread allocate and free while another one captures a stream: an object may be collected at any time, and
+// what it frees is no part of the graph.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 template <class S, int FAM>
 int strain_launch(const lbm355_sweep_desc* d, const void* pdf, const double* tab, double* out, double omega,
                   int last, hipStream_t s) {
@@ -493,6 +501,23 @@ int lbm355_get_macroscopic(const lbm355_sweep_desc* d, const void* pdf, double* 
   out.scalar_stride[2] = out.vector_stride[2] = d->out_stride_z;
   out.vector_stride[3] = d->out_stride_c;
   return lbm355_get_fields(d, pdf, &out, last_pattern, stream);
+}
+
+void* lbm355_host_alloc(int64_t bytes) {
+  const RelaxedCapture relaxed;
+  void* p = nullptr;
+  if (bytes <= 0 || hipHostMalloc(&p, (size_t)bytes, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();   // the caller's answer to NULL is pageable memory
+    return nullptr;
+  }
+  return p;
+}
+
+int lbm355_host_free(void* memory) {
+  const RelaxedCapture relaxed;
+  if (hipHostFree(memory) == hipSuccess) return LBM355_OK;
+  (void)hipGetLastError();
+  return fail2(LBM355_ERR_ARG, "not memory of lbm355_host_alloc");
 }
 
 int lbm355_get_strain_rate(const lbm355_sweep_desc* d, const void* pdf, const double* table_f64, double* strain_rate,

@@ -108,12 +108,15 @@ class LatticeBoltzmannStep:
         dt = config.data_type
         self._src = create_pdf_array(domain_size, q, 1, dt)
         self._tmp = create_pdf_array(domain_size, q, 1, dt) if self._two_arrays else None
-        # macroscopic fields: host numpy (interior) + FP64 device staging with the PDF ghost layout
-        # (pinned memory, which the getter's kernel writes directly)
-        self._rho_pinned = torch.ones(domain_size, dtype=torch.float64, pin_memory=True)
-        self._u_pinned = torch.zeros(domain_size + (dim,), dtype=torch.float64, pin_memory=True)
-        self._rho_host = self._rho_pinned.numpy()
-        self._u_host = self._u_pinned.numpy()
+        # macroscopic fields: host numpy (interior) + FP64 device staging with the PDF ghost layout.  The host fields are
+        # pinned, for the getter's kernel to write directly, unless there is no such memory to be had.
+        fields = [nat.pinned_array(domain_size), nat.pinned_array(domain_size + (dim,))]
+        self._host_pinned = all(f is not None for f in fields)
+        if not self._host_pinned:
+            fields = [np.empty(domain_size), np.empty(domain_size + (dim,))]
+        self._rho_host, self._u_host = fields
+        self._rho_host.fill(1.0)
+        self._u_host.fill(0.0)
         self._rho_dev = torch.zeros([n + 2 for n in domain_size][::-1], dtype=torch.float64, device="cuda")
         self._u_dev = torch.zeros([dim] + [n + 2 for n in domain_size][::-1], dtype=torch.float64, device="cuda")
         self._boundary_handling = LatticeBoltzmannBoundaryHandling.for_domain(self.method, domain_size,
@@ -212,8 +215,8 @@ class LatticeBoltzmannStep:
         D = self.dim
         inner = (slice(1, -1),) * D
         back = tuple(range(D - 1, -1, -1))
-        self._rho_dev[inner] = self._rho_pinned.cuda(non_blocking=True).permute(*back)
-        self._u_dev[(slice(None),) + inner] = self._u_pinned.cuda(non_blocking=True).permute(D, *back)
+        self._rho_dev[inner] = torch.from_numpy(self._rho_host).cuda(non_blocking=True).permute(*back)
+        self._u_dev[(slice(None),) + inner] = torch.from_numpy(self._u_host).cuda(non_blocking=True).permute(D, *back)
         d = self._descriptor()
         tab, _ = method_table(self.method, self.kernel_params, np.float64,
                               corrections=self._kernels[0].corrections)
@@ -261,17 +264,22 @@ class LatticeBoltzmannStep:
         # MI355X 96^3 (28 MB) takes 0.56 ms, 50 GB/s, where pageable copies of x-fastest fields and numpy's transposition
         # took 12 ms; 40x80 takes 18 us.  (Staging on the device and one copy is 16 us slower there, and 7% faster at best
         # above 30 MB.)
+        host = [torch.from_numpy(self._rho_host), torch.from_numpy(self._u_host)]
+        rho, u = host if self._host_pinned else (torch.empty_like(f, device="cuda") for f in host)
         out = nat.MacroscopicOut()
         out.dtype = nat.F64
-        out.density = self._rho_pinned.data_ptr()
-        out.velocity = self._u_pinned.data_ptr()
+        out.density = rho.data_ptr()
+        out.velocity = u.data_ptr()
         D = self.dim
         for a in range(D):
-            out.scalar_stride[a] = self._rho_pinned.stride(a)
-            out.vector_stride[a] = self._u_pinned.stride(a)
-        out.vector_stride[3] = self._u_pinned.stride(D)
+            out.scalar_stride[a] = rho.stride(a)
+            out.vector_stride[a] = u.stride(a)
+        out.vector_stride[3] = u.stride(D)
         nat.check(nat.load().lbm355_get_fields(ctypes.byref(d), ctypes.c_void_p(self._src.data_ptr()),
                                                ctypes.byref(out), last, nat.current_stream_handle()))
+        if not self._host_pinned:
+            host[0].copy_(rho)
+            host[1].copy_(u)
         torch.cuda.current_stream().synchronize()
 
     # ------------------------------------------------------------------ fixed two-step loop
