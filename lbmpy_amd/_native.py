@@ -5,12 +5,9 @@ resolves to the HIP runtime torch already loaded: PDF tensors, streams and the
 kernels then live in one runtime.  There is no fallback: if the library is
 missing the import raises.
 """
-import collections
 import ctypes
 import os
-import weakref
 
-import numpy as np
 import torch  # noqa: F401  (must precede the library load, see module docstring)
 
 from .csrc.build import library_path, source_hash
@@ -207,31 +204,3 @@ def check(rc):
 
 def current_stream_handle():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-
-
-_freed_later = collections.deque()
-
-
-def _free_pinned(lib, address):
-    """Gives pinned memory back, or notes it for the next call where this thread's stream is being captured (the free
-    waits for the GPU)."""
-    _freed_later.append(address)
-    if not torch.cuda.is_current_stream_capturing():
-        while _freed_later:
-            try:
-                lib.lbm355_host_free(_freed_later.popleft())
-            except IndexError:              # another thread was faster
-                return
-
-
-def pinned_array(shape):
-    """An FP64 numpy array in pinned host memory of exactly its size, which is given back when the array and all its
-    views are gone; None where there is none to be had."""
-    lib = load()
-    nbytes = 8 * int(np.prod(shape, dtype=np.int64))
-    address = lib.lbm355_host_alloc(nbytes)
-    if not address:
-        return None
-    memory = (ctypes.c_char * nbytes).from_address(address)
-    weakref.finalize(memory, _free_pinned, lib, address).atexit = False
-    return np.frombuffer(memory, dtype=np.float64).reshape(shape)

@@ -28,6 +28,7 @@ from . import _native as nat
 from .boundaries import LatticeBoltzmannBoundaryHandling
 from .creationfunctions import (update_with_default_parameters, create_lb_function, Timestep, CreateKernelConfig)
 from .enums import Stencil, Target
+from .host_memory import pinned_array
 from .kernel_tables import method_table
 from .stencils import LBStencil
 from .sweep import create_pdf_array, TORCH_DTYPES
@@ -110,7 +111,7 @@ class LatticeBoltzmannStep:
         self._tmp = create_pdf_array(domain_size, q, 1, dt) if self._two_arrays else None
         # macroscopic fields: host numpy (interior) + FP64 device staging with the PDF ghost layout.  The host fields are
         # pinned, for the getter's kernel to write directly, unless there is no such memory to be had.
-        fields = [nat.pinned_array(domain_size), nat.pinned_array(domain_size + (dim,))]
+        fields = [pinned_array(domain_size), pinned_array(domain_size + (dim,))]
         self._host_pinned = all(f is not None for f in fields)
         if not self._host_pinned:
             fields = [np.empty(domain_size), np.empty(domain_size + (dim,))]
