@@ -214,10 +214,16 @@ class LatticeBoltzmannStep:
     def set_pdf_fields_from_macroscopic_values(self):
         """Equilibrium from the host density/velocity fields (lbstep.py:268-269), on the GPU."""
         D = self.dim
-        inner = (slice(1, -1),) * D
+        inner = (slice(1, -1),) * (D - 1)
         back = tuple(range(D - 1, -1, -1))
-        self._rho_dev[inner] = torch.from_numpy(self._rho_host).cuda(non_blocking=True).permute(*back)
-        self._u_dev[(slice(None),) + inner] = torch.from_numpy(self._u_host).cuda(non_blocking=True).permute(D, *back)
+        nx = self._domain_size[0]
+        # planes of x at a time, so that the copies on the way take at most 64 MiB of device memory (or a plane)
+        planes = max(1, (64 << 20) * nx // (8 * D * self.number_of_cells))
+        for x in range(0, nx, planes):
+            at = inner + (slice(1 + x, 1 + min(x + planes, nx)),)
+            self._rho_dev[at] = torch.from_numpy(self._rho_host[x:x + planes]).cuda(non_blocking=True).permute(*back)
+            self._u_dev[(slice(None),) + at] = \
+                torch.from_numpy(self._u_host[x:x + planes]).cuda(non_blocking=True).permute(D, *back)
         d = self._descriptor()
         tab, _ = method_table(self.method, self.kernel_params, np.float64,
                               corrections=self._kernels[0].corrections)

@@ -123,3 +123,20 @@ def test_native_allocation_refuses_nonsense():
     p = lib.lbm355_host_alloc(1000)
     assert p and lib.lbm355_host_free(p) == 0
     assert float((torch.ones(4, device="cuda") * 2).sum()) == 8.0
+
+
+def test_setting_the_fields_takes_bounded_device_memory():
+    shape = (300, 160, 120)                # 138 MB of velocity: three parts, the last one smaller
+    s = _step(shape)
+    every = (slice(None),) * 3
+    rho0, u0 = s.density_slice(every, masked=False).copy(), s.velocity_slice(every, masked=False).copy()
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    s.set_pdf_fields_from_macroscopic_values()
+    # a part of velocity, and one of density a third its size, each once more where the last is not yet collected
+    assert torch.cuda.max_memory_allocated() - before <= 2 * (64 << 20)
+    s.post_run()
+    # set and read back in FP64 (the populations' type): 19 terms of at most 1/3
+    np.testing.assert_allclose(s.density_slice(every, masked=False), rho0, rtol=0, atol=1e-14)
+    np.testing.assert_allclose(s.velocity_slice(every, masked=False), u0, rtol=0, atol=1e-14)
