@@ -480,12 +480,18 @@ int validate(const lbm355_sweep_desc* d) {
   return LBM355_OK;
 }
 
-// AA odd streams its populations only by rows: it reaches none but the centre's at the cell itself.
+// AA odd streams its populations only by rows: it reaches none but the centre's at the cell itself.  The FP16 moment and
+// central-moment kernels, which have no row form, keep y and z in scalar registers where a block is a row (AA 256^3, us a
+// launch with consecutive cells and so: D3Q19 TRT 233 and 223, D3Q27 TRT 354 and 349, D3Q19 central 252 and 250, D3Q27
+// central 382 and 377; D3Q19 TRT 192^3 96 and 93).  Rows of two blocks, 483 and 490 at 512x256x256, walls, D3Q27 TRT 359 and
+// 367, and the cumulants, 320 and 323, lose by it.
 StreamedModes streamed_modes(const lbm355_sweep_desc* d, size_t* row_lds) {
   const bool waves = d->nx % 64 == 0;
   if (table_pattern(d->pattern)) return {lbm355_eso_row_lds(d, row_lds), waves, false};
-  const bool odd = d->pattern == LBM355_AA_ODD;
-  return {use_rowlds(d, row_lds), waves && !odd, !odd};
+  if (d->pattern == LBM355_AA_ODD)
+    return {use_rowlds(d, row_lds),
+            waves && d->nx <= 256 && !has_walls(d) && odd_waves_kernel(d->family, d->store_dtype), false};
+  return {use_rowlds(d, row_lds), waves, true};
 }
 
 template <class TC>

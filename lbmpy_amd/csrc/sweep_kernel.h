@@ -139,8 +139,13 @@ __global__ void __launch_bounds__(MODE == ACCESS_ROWS ? 512 : 256) sweep_kernel(
   }
 }
 
+// Whether AA odd has a kernel of ACCESS_WAVES, without walls (streamed_modes in sweep.hip).
+constexpr bool odd_waves_kernel(int family, int store) {
+  return store == LBM355_F16 && (family == LBM355_FAMILY_MOMENT || family == LBM355_FAMILY_CENTRAL);
+}
+
 // AA even has no x-shifts (no row kernel); AA odd reaches no population but the centre's at the cell itself, so its
-// per-cell kernel is the ACCESS_CACHED one.
+// per-cell kernel is the ACCESS_CACHED one, but for odd_waves_kernel's.
 template <class S, int FAM, bool WALLS, class TS, class TC>
 void* pick_walls(int pat, int mode) {
 #define LBM_K(P, M) (void*)sweep_kernel<S, FAM, P, WALLS, M, TS, TC>
@@ -149,6 +154,8 @@ void* pick_walls(int pat, int mode) {
     if (mode == ACCESS_WAVES) return LBM_K(LBM355_PULL, ACCESS_WAVES);
     return mode == ACCESS_LINES ? LBM_K(LBM355_PULL, ACCESS_LINES) : LBM_K(LBM355_PULL, ACCESS_CACHED);
   }
+  if constexpr (!WALLS && odd_waves_kernel(FAM, sizeof(TS) == 2 ? LBM355_F16 : LBM355_F32))
+    if (pat == LBM355_AA_ODD && mode == ACCESS_WAVES) return LBM_K(LBM355_AA_ODD, ACCESS_WAVES);
   if (pat == LBM355_AA_ODD) return mode == ACCESS_ROWS ? LBM_K(LBM355_AA_ODD, ACCESS_ROWS) : LBM_K(LBM355_AA_ODD, ACCESS_CACHED);
   return nullptr;
 #undef LBM_K

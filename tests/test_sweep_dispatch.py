@@ -24,10 +24,10 @@ def lib():
     return nat.load()
 
 
-def _mode(lib, stencil, pattern, dtype, shape, g=0, walls=False, pad=0, shift=0, closure=False):
+def _mode(lib, stencil, pattern, dtype, shape, g=0, walls=False, pad=0, shift=0, closure=False, cumulant=False):
     d = nat.SweepDesc()
     d.stencil, q = STENCILS[stencil]
-    d.family = nat.FAMILY_CUMULANT if closure else nat.FAMILY_MOMENT
+    d.family = nat.FAMILY_CUMULANT if closure or cumulant else nat.FAMILY_MOMENT
     d.pattern, d.store_dtype = PATTERNS[pattern], TYPES[dtype]
     d.compute_dtype = nat.F64 if dtype == "f64" else nat.F32
     shape = tuple(shape) + (1,) * (3 - len(shape))
@@ -62,8 +62,9 @@ def _mode(lib, stencil, pattern, dtype, shape, g=0, walls=False, pad=0, shift=0,
     (("D3Q27", "even", "f32", (200, 224, 224)), LINES), (("D3Q27", "odd", "f32", (200, 224, 224)), SHARED),
     (("D3Q27", "esotwist", "f32", (192, 256, 224)), ROWS), (("D3Q27", "esopull", "f32", (576, 144, 128)), WAVES),
     (("D3Q27", "esopull", "f32", (200, 224, 224)), SHARED), (("D3Q27", "push", "f32", (256, 192, 160)), ROWS),
-    # FP16 has no row kernels for pull and AA
-    (("D3Q27", "odd", "f16", (256, 256, 256)), SHARED), (("D3Q27", "even", "f16", (256, 256, 256)), WAVES),
+    # FP16 has no row kernels for pull and AA; a block a row in AA odd
+    (("D3Q27", "odd", "f16", (256, 256, 256)), WAVES), (("D3Q19", "odd", "f16", (512, 256, 256)), SHARED),
+    (("D3Q19", "odd", "f16", (250, 200, 180)), SHARED), (("D3Q27", "even", "f16", (256, 256, 256)), WAVES),
     (("D3Q19", "pull", "f16", (123, 96, 192)), LINES), (("D3Q27", "esotwist", "f16", (256, 256, 256)), ROWS),
     # two dimensions
     (("D2Q9", "pull", "f64", (512, 4096)), ROWS), (("D2Q9", "pull", "f64", (1024, 1024)), WAVES),
@@ -89,6 +90,8 @@ def test_alignment_walls_and_padding(lib):
     for n, pattern, want in ((128, "odd", CACHED), (192, "even", SHARED), (256, "even", WAVES), (256, "odd", ROWS)):
         assert _mode(lib, "D3Q27", pattern, "f32", (n, n, n), closure=True) == want
     assert _mode(lib, "D3Q27", "even", "f32", (200, 128, 128), closure=True) < 0
+    for kw in (dict(cumulant=True), dict(walls=True)):
+        assert _mode(lib, "D3Q27", "odd", "f16", (256, 256, 256), **kw) == SHARED
 
 
 def test_cases_of_the_large_domain_tests(lib):
