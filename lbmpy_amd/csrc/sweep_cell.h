@@ -432,18 +432,23 @@ inline bool backwards_sweep(int pattern, const void* src, const void* dst) {
   return src != dst && (uintptr_t)src < (uintptr_t)dst;
 }
 inline bool meets_cached(int64_t bytes, bool in_place) { return in_place || bytes <= 8 * HALF_CACHE_BYTES; }
-// Whether that is worth regular accesses where the lines would allow non-temporal ones: D3Q27 cumulant AA FP32 160^3,
-// 442 MB, 151 (151) streamed and 132 (151) so, 192^3, 764 MB, 276 (276) and 248 (266), but 224^3, 1.2 GB, 438 (437) and
-// 433 (444); FP64 128^3 161 (162) and 136 (158); EsoTwist FP32 150x150x160 147 (151) and 125 (135).  With walls arrays in
-// turn lose (D3Q19 TRT 200x200x160 156 (156) and 152 (165)), FP16 too (200^3 146 (145) and 134 (153)), and two arrays
-// gain nothing (D3Q19 TRT pull 160^3 119 (119) and 117 (118)).
-inline bool cached_anyway(int64_t bytes, int store, bool in_place, bool walls) {
-  return in_place && !walls && store != LBM355_F16 && bytes <= 6 * HALF_CACHE_BYTES;
-}
 inline bool has_walls(const lbm355_sweep_desc* d) {
   for (int a = 0; a < (d->stencil == LBM355_D2Q9 ? 2 : 3); ++a)
     if (d->face[a] == LBM355_FACE_NOSLIP) return true;
   return false;
+}
+// Whether that is worth regular accesses where the lines would allow non-temporal ones: D3Q27 cumulant AA FP32 160^3,
+// 442 MB, 151 (151) streamed and 132 (151) so, 192^3, 764 MB, 276 (276) and 248 (266), but 224^3, 1.2 GB, 438 (437) and
+// 433 (444); FP64 128^3 161 (162) and 136 (158); EsoTwist FP32 150x150x160 147 (151) and 125 (135).  With walls arrays in
+// turn lose (D3Q19 TRT 200x200x160 156 (156) and 152 (165)), FP16 too (200^3 146 (145) and 134 (153)), and two arrays
+// gain nothing (D3Q19 TRT pull 160^3 119 (119) and 117 (118)).  Fewer populations gain less at the upper end: D3Q19 TRT AA
+// 192x192x208, 583 MB, 210 (210) and 189 (202), 256x192x192, 717 MB, 242 (241) and 238 (248), and D2Q9 AA, up to 576 MiB,
+// FP32 3520^2, 446 MB, 143 (143) and 135 (145), but 4096^2, 604 MB, 193 (194) and 196 (215), FP64 3072^2, 679 MB, 221 (221)
+// and 220 (235).
+inline bool cached_anyway(const lbm355_sweep_desc* d, int64_t bytes, bool in_place) {
+  const bool flat_aa = d->stencil == LBM355_D2Q9 && !table_pattern(d->pattern);
+  return in_place && !has_walls(d) && d->store_dtype != LBM355_F16 &&
+         (flat_aa ? 2 * bytes < 9 * HALF_CACHE_BYTES : bytes <= 6 * HALF_CACHE_BYTES);
 }
 
 // The streamed modes that a sweep has a kernel for.
@@ -465,7 +470,7 @@ inline AccessMode choose_access(const lbm355_sweep_desc* d, const void* src, con
   const bool in_place = src == dst;
   const int64_t bytes = population_bytes(d, in_place);
   if (fits_cache(bytes, d->store_dtype, in_place)) return ACCESS_CACHED;
-  if (!cached_anyway(bytes, d->store_dtype, in_place, has_walls(d)) && starts_lines(d, src, dst)) {
+  if (!cached_anyway(d, bytes, in_place) && starts_lines(d, src, dst)) {
     if (m.rows) return ACCESS_ROWS;
     if (m.waves) return ACCESS_WAVES;
     if (m.lines) return ACCESS_LINES;

@@ -69,7 +69,10 @@ def _mode(lib, stencil, pattern, dtype, shape, g=0, walls=False, pad=0, shift=0,
     # two dimensions
     (("D2Q9", "pull", "f64", (512, 4096)), ROWS), (("D2Q9", "pull", "f64", (1024, 1024)), WAVES),
     (("D2Q9", "pull", "f64", (1000, 1024)), LINES), (("D2Q9", "pull", "f64", (1000, 1001)), SHARED),
-    (("D2Q9", "odd", "f64", (448, 32768)), ROWS), (("D2Q9", "even", "f32", (4096, 8192)), WAVES),
+    # in place up to 576 MiB
+    (("D2Q9", "even", "f32", (4000, 4000)), SHARED), (("D2Q9", "even", "f32", (4096, 4096)), WAVES),
+    (("D2Q9", "odd", "f64", (512, 14000)), SHARED), (("D2Q9", "odd", "f64", (512, 16400)), ROWS),
+    (("D2Q9", "esopull", "f32", (4096, 4096)), SHARED), (("D2Q9", "odd", "f64", (448, 32768)), ROWS), (("D2Q9", "even", "f32", (4096, 8192)), WAVES),
 ])
 def test_chosen_mode(lib, args, want):
     assert _mode(lib, *args) == want
