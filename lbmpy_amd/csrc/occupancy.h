@@ -48,7 +48,8 @@ inline size_t lds_for_wave_cap(int waves, unsigned block_threads, size_t kernel_
 // 0.635 -> 0.607, EsoTwist 0.634 -> 0.604, EsoPull 0.622 -> 0.599, EsoPush 0.617 -> 0.594, push 0.644 -> 0.605;
 // of D3Q19 SRT / TRT / MRT: pull 0.425 -> 0.415, AA even 0.431 -> 0.415, AA odd 0.424 -> 0.413, the Eso patterns
 // 0.423-0.434 -> 0.409-0.419, push 0.437 -> 0.421.  Caps that gained less than about 1.5% are left out.
-// One wave per SIMD is slower everywhere.
+// One wave per SIMD is slower everywhere.  The FP16 kernels take 64 and 72 registers (8 and 7 waves by themselves); on
+// lines of no whole rows (250x200x180) their caps gain 208 -> 195 us in the odd sweep and cost 161 -> 167 in the even one.
 enum CapKind { CAP_PULL, CAP_AA_EVEN, CAP_AA_ODD, CAP_ESOTWIST, CAP_ESOPULL, CAP_ESOPUSH, CAP_PUSH, CAP_KINDS };
 
 struct WaveCaps {
@@ -59,7 +60,7 @@ struct WaveCaps {
 constexpr WaveCaps kWaveCaps[] = {
     {LBM355_FAMILY_CUMULANT, LBM355_D3Q27, LBM355_F32, {3, 3, 2, 2, 2, 2, 2}},
     {LBM355_FAMILY_CUMULANT, LBM355_D3Q27, LBM355_F64, {0, 2, 2, 0, 0, 0, 0}},  // AA: 1.337 / 1.344 -> 1.272 / 1.240
-    {LBM355_FAMILY_CUMULANT, LBM355_D3Q27, LBM355_F16, {0, 4, 4, 0, 0, 0, 0}},  // AA: 0.334 / 0.329 -> 0.316 / 0.316
+    {LBM355_FAMILY_CUMULANT, LBM355_D3Q27, LBM355_F16, {0, 4, 4, 0, 0, 0, 0}},  // AA: 0.327 / 0.342 -> 0.323 / 0.328
     {LBM355_FAMILY_MOMENT, LBM355_D3Q19, LBM355_F32, {4, 3, 4, 4, 4, 4, 3}},
     {LBM355_FAMILY_MOMENT, LBM355_D3Q27, LBM355_F32, {4, 3, 0, 0, 0, 0, 0}},  // pull 0.622->0.605, even 0.618->0.596
     {LBM355_FAMILY_CENTRAL, LBM355_D3Q19, LBM355_F32, {0, 0, 3, 3, 3, 0, 0}},  // AA odd 0.435 -> 0.415, Eso 1.7%

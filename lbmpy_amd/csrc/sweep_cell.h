@@ -393,7 +393,7 @@ inline bool starts_lines(const lbm355_sweep_desc* d, const void* src, const void
 // D3Q27 cumulant FP32 AA unless noted, every step on the same array:
 // - What fits the Infinity Cache (fits_cache) is found there by the next step, if it was written with regular stores:
 //   64^3 13.1 -> 10.0, 128^3 81.8 -> 56.7, 128^3 with ghost layers 145 -> 61, EsoTwist 100x90x80 28.2 -> 23.5, D3Q19 TRT
-//   pull 128x128x96 43.6 -> 33.0.  One run of blocks per XCD keeps a cell's neighbours in its L2 as well: D3Q19 SRT
+//   pull 96x96x80 (112 MB) 24.1 -> 21.5.  One run of blocks per XCD keeps a cell's neighbours in its L2 as well: D3Q19 SRT
 //   FP64 64x32x32 9.8 -> 6.4.  (The row kernel with regular accesses gave 61.2 at 128^3.)
 // - Above that, lines that start with a wavefront are best streamed past the caches, as they come: 256^3 593 (685 with
 //   regular accesses, 640 with runs of 16 blocks per XCD), FP16 250x200x180 252 -> 170.
@@ -406,8 +406,8 @@ constexpr int64_t SMALL_CELLS = 1 << 18;   // below: blocks of one wavefront, to
 
 // Whether the populations' bytes fit the 256 MiB Infinity Cache to a gain.  In place in FP32 or FP64 they may fill it:
 // at 128^3 (216 MiB) regular accesses win also for a program that takes three such arrays in turn (82 -> 71 us, one
-// array 57; learned closure 107 -> 79, three in turn 106 -> 96).  Two arrays and FP16 storage lose more to such turns
-// than they gain alone (pull D3Q19 128x128x80, 253 MB: 36.7 -> 29.9 us for one pair of arrays, 42.5 for three in turn;
+// array 57; learned closure 120 -> 90, three in turn 108 -> 101).  Two arrays and FP16 storage lose more to such turns
+// than they gain alone (pull D3Q19 128x128x80, 199 MB: 39.3 -> 33.8 us for one pair of arrays, three in turn 38.3 -> 40.9;
 // FP16 192x128x128, 162 MiB: 54.7 -> 49.5, 63.5): they may fill half of it, where they do not.
 inline int64_t population_bytes(const lbm355_sweep_desc* d, bool in_place) {
   const int64_t es = d->store_dtype == LBM355_F64 ? 8 : (d->store_dtype == LBM355_F32 ? 4 : 2);
@@ -439,7 +439,7 @@ inline bool has_walls(const lbm355_sweep_desc* d) {
 }
 // Whether that is worth regular accesses where the lines would allow non-temporal ones: D3Q27 cumulant AA FP32 160^3,
 // 442 MB, 151 (151) streamed and 132 (151) so, 192^3, 764 MB, 276 (276) and 248 (266), but 224^3, 1.2 GB, 438 (437) and
-// 433 (444); FP64 128^3 161 (162) and 136 (158); EsoTwist FP32 150x150x160 147 (151) and 125 (135).  With walls arrays in
+// 433 (444); FP64 128^3 161 (162) and 136 (158); EsoTwist FP32 192x128x128 127 (125) and 108 (114).  With walls arrays in
 // turn lose (D3Q19 TRT 200x200x160 156 (156) and 152 (165)), FP16 too (200^3 146 (145) and 134 (153)), and two arrays
 // gain nothing (D3Q19 TRT pull 160^3 119 (119) and 117 (118)).  Fewer populations gain less at the upper end: D3Q19 TRT AA
 // 192x192x208, 583 MB, 210 (210) and 189 (202), 256x192x192, 717 MB, 242 (241) and 238 (248), and D2Q9 AA, up to 576 MiB,
