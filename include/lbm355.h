@@ -237,6 +237,11 @@ typedef struct lbm355_macroscopic_out {
 int lbm355_get_fields(const lbm355_sweep_desc* desc, const void* pdf, const lbm355_macroscopic_out* out,
                       int32_t last_pattern, void* stream);
 
+/* Whether every element that lbm355_get_fields would write is its own: the fields share no memory with the populations,
+ * nor with each other (its threads write in no order).  Components interleaved per cell in one array do not share.  1 or
+ * 0; nothing is read or written through the pointers. */
+int32_t lbm355_fields_apart(const lbm355_sweep_desc* desc, const void* pdf, const lbm355_macroscopic_out* out);
+
 /* Pinned host memory, of exactly `bytes` and given back by the free (which first waits for the GPU); NULL if there is
  * none to be had.  The free returns an error for a pointer that is not of the allocation's. */
 void* lbm355_host_alloc(int64_t bytes);

@@ -67,8 +67,8 @@ ACCESS_ROWS, ACCESS_WAVES, ACCESS_LINES, ACCESS_CACHED, ACCESS_SHARED = 0, 1, 2,
 
 EXPORTED = ("lbm355_sweep", "lbm355_sweep_access", "lbm355_sweep_with_access", "lbm355_table_elements",
             "lbm355_noslip_links", "lbm355_reduce_conserved", "lbm355_count_nonfinite",
-            "lbm355_set_equilibrium", "lbm355_get_macroscopic", "lbm355_get_fields", "lbm355_stream_copy", "lbm355_desc_size",
-            "lbm355_last_error", "lbm355_version", "lbm355_batch_create", "lbm355_batch_sweep",
+            "lbm355_set_equilibrium", "lbm355_get_macroscopic", "lbm355_get_fields", "lbm355_fields_apart",
+            "lbm355_stream_copy", "lbm355_desc_size", "lbm355_last_error", "lbm355_version", "lbm355_batch_create", "lbm355_batch_sweep",
             "lbm355_batch_info", "lbm355_batch_destroy", "lbm355_batch_sweep_static", "lbm355_closure_params_size",
             "lbm355_closure_master_size", "lbm355_closure_features", "lbm355_closure_forward",
             "lbm355_closure_train_step", "lbm355_closure_adam", "lbm355_closure_workspace_floats",
@@ -114,6 +114,8 @@ def load(path=None):
     lib.lbm355_get_fields.argtypes = [ctypes.POINTER(SweepDesc), c_void_p, ctypes.POINTER(MacroscopicOut), c_int32,
                                       c_void_p]
     lib.lbm355_get_fields.restype = c_int32
+    lib.lbm355_fields_apart.argtypes = [ctypes.POINTER(SweepDesc), c_void_p, ctypes.POINTER(MacroscopicOut)]
+    lib.lbm355_fields_apart.restype = c_int32
     lib.lbm355_host_alloc.argtypes = [c_int64]
     lib.lbm355_host_alloc.restype = c_void_p
     lib.lbm355_host_free.argtypes = [c_void_p]

@@ -419,6 +419,34 @@ struct RelaxedCapture {
   ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
 
+// Whether n strides each go beyond what the smaller ones reach, so that no two indices meet.
+bool nested(const int64_t* size, const int64_t* stride, int n) {
+  int order[4], k = 0;
+  for (int a = 0; a < n; ++a)
+    if (size[a] > 1) {
+      int at = k++;
+      for (; at > 0 && stride[order[at - 1]] > stride[a]; --at) order[at] = order[at - 1];
+      order[at] = a;
+    }
+  int64_t reach = 1;
+  for (int j = 0; j < k; ++j) {
+    if (stride[order[j]] < reach) return false;
+    reach = stride[order[j]] * size[order[j]];
+  }
+  return true;
+}
+
+struct Span {
+  uintptr_t first, end;
+  bool apart(const Span& o) const { return first >= o.end || o.first >= end; }
+};
+
+Span span_of(const void* p, size_t element, const int64_t* size, const int64_t* stride, int n) {
+  int64_t last = 0;
+  for (int a = 0; a < n; ++a) last += (size[a] - 1) * stride[a];
+  return {(uintptr_t)p, (uintptr_t)p + element * (size_t)(last + 1)};
+}
+
 template <class S, int FAM>
 int strain_launch(const lbm355_sweep_desc* d, const void* pdf, const double* tab, double* out, double omega,
                   int last, hipStream_t s) {
@@ -486,6 +514,59 @@ int lbm355_get_fields(const lbm355_sweep_desc* d, const void* pdf, const lbm355_
   if (d->stencil == LBM355_D3Q19) return get_dtype<D3Q19>(d, pdf, *out, last_pattern, s);
   if (d->stencil == LBM355_D3Q27) return get_dtype<D3Q27>(d, pdf, *out, last_pattern, s);
   return fail2(LBM355_ERR_ARG, "unknown stencil");
+}
+
+int32_t lbm355_fields_apart(const lbm355_sweep_desc* d, const void* pdf, const lbm355_macroscopic_out* out) {
+  if (!d || !pdf || !out) return 0;
+  const int D = d->stencil == LBM355_D2Q9 ? 2 : 3;
+  const int Q = d->stencil == LBM355_D2Q9 ? 9 : (d->stencil == LBM355_D3Q19 ? 19 : 27);
+  const size_t es = out->dtype == LBM355_F32 ? 4 : 8;
+  const int64_t g2 = 2 * d->ghost_layers, size[4] = {d->nx, d->ny, D == 3 ? d->nz : D, D};
+  const int64_t psize[4] = {d->nx + g2, d->ny + g2, D == 3 ? d->nz + g2 : 1, Q};
+  const int64_t pstride[4] = {1, d->stride_y, d->stride_z, d->stride_q};
+  const Span populations =
+      span_of(pdf, d->store_dtype == LBM355_F64 ? 8 : (d->store_dtype == LBM355_F32 ? 4 : 2), psize, pstride, 4);
+  int64_t vector_stride[4] = {out->vector_stride[0], out->vector_stride[1], out->vector_stride[2], out->vector_stride[3]};
+  if (D == 2) vector_stride[2] = out->vector_stride[3];
+  Span spans[3];
+  uintptr_t at[5];
+  int fields = 0, components = 0;
+  const int64_t* cells = nullptr;
+  bool same_cells = true, apart = true;
+  const void* scalars[2] = {out->density, out->density_deviation};
+  for (const void* p : scalars) {
+    if (!p) continue;
+    if (!nested(size, out->scalar_stride, D)) return 0;
+    cells = out->scalar_stride;
+    spans[fields++] = span_of(p, es, size, out->scalar_stride, D);
+    at[components++] = (uintptr_t)p;
+  }
+  if (out->velocity) {
+    if (!nested(size, vector_stride, D + 1)) return 0;
+    if (cells)
+      for (int a = 0; a < D; ++a) same_cells = same_cells && cells[a] == vector_stride[a];
+    cells = vector_stride;
+    spans[fields++] = span_of(out->velocity, es, size, vector_stride, D + 1);
+    for (int c = 0; c < D; ++c) at[components++] = (uintptr_t)out->velocity + es * c * (uintptr_t)out->vector_stride[3];
+  }
+  for (int k = 0; k < fields; ++k) {
+    if (!spans[k].apart(populations)) return 0;
+    for (int l = 0; l < k; ++l) apart = apart && spans[k].apart(spans[l]);
+  }
+  if (apart) return 1;
+  // one set of cell strides, and all components of a cell within the smallest of them
+  int64_t smallest = INT64_MAX;
+  for (int a = 0; a < D; ++a)
+    if (size[a] > 1 && cells[a] < smallest) smallest = cells[a];
+  if (!same_cells || smallest == INT64_MAX || !nested(size, cells, D)) return 0;
+  uintptr_t low = at[0], high = at[0];
+  for (int k = 0; k < components; ++k) {
+    low = at[k] < low ? at[k] : low;
+    high = at[k] > high ? at[k] : high;
+    for (int l = 0; l < k; ++l)
+      if (at[k] == at[l]) return 0;
+  }
+  return high - low < es * (uintptr_t)smallest;
 }
 
 int lbm355_get_macroscopic(const lbm355_sweep_desc* d, const void* pdf, double* density, double* velocity,

@@ -165,45 +165,6 @@ def _set(ctx, pdfs, density, velocity, code):
                                          nat.current_stream_handle()))
 
 
-def _own_memory(pdfs, scalars, velocity):
-    """Whether every element that the getter writes is its own: the fields share no memory with the populations, nor
-    with each other (a kernel's threads write in no order).  Fields interleaved per cell in one array do not share."""
-    def nested(sizes, strides):             # each stride beyond what the smaller ones reach
-        reach = 1
-        for s, n in sorted(zip(strides, sizes)):
-            if n > 1:
-                if s < reach:
-                    return False
-                reach = s * n
-        return True
-
-    def span(t):
-        return t.data_ptr(), t.data_ptr() + t.element_size() * (1 + sum((n - 1) * s for n, s in zip(t.shape, t.stride())))
-
-    def apart(a, b):
-        return a[0] >= b[1] or b[0] >= a[1]
-
-    fields = scalars + ([velocity] if velocity is not None else [])
-    if not all(nested(t.shape, t.stride()) for t in fields):
-        return False
-    if len({t.untyped_storage().data_ptr() for t in fields + [pdfs]}) == len(fields) + 1:
-        return True
-    spans = [span(t) for t in fields]
-    if not all(apart(s, span(pdfs)) for s in spans):
-        return False
-    if all(apart(a, b) for k, a in enumerate(spans) for b in spans[:k]):
-        return True
-    # one set of cell strides, and all components of a cell within the smallest of them
-    D = pdfs.dim() - 1
-    at = [t.data_ptr() for t in scalars]
-    if velocity is not None:
-        at += [velocity.data_ptr() + velocity.element_size() * velocity.stride(D) * c for c in range(velocity.shape[D])]
-    cells, sizes = fields[0].stride()[:D], fields[0].shape[:D]
-    smallest = min((s for s, n in zip(cells, sizes) if n > 1), default=0) * fields[0].element_size()
-    return all(t.stride()[:D] == cells for t in fields) and nested(sizes, cells) and \
-        len(set(at)) == len(at) and max(at) - min(at) < smallest
-
-
 def _get_in_place(ctx, pdfs, density, velocity, code, density_deviation):
     """The getter straight into the output tensors; False where they do not admit it (the kernel takes plain FP64 and FP32
     fields of any order, shaped like the PDFs, that torch would write without further bookkeeping)."""
@@ -215,8 +176,7 @@ def _get_in_place(ctx, pdfs, density, velocity, code, density_deviation):
                and not t.is_neg() and not t.is_inference() for t in fields) or \
             len({t.dtype for t in fields}) != 1 or fields[0].dtype not in (torch.float64, torch.float32) or \
             any(tuple(t.shape) != spatial for t in scalars) or len({t.stride() for t in scalars}) > 1 or \
-            (velocity is not None and tuple(velocity.shape) != spatial + (D,)) or \
-            not _own_memory(pdfs, scalars, velocity):
+            (velocity is not None and tuple(velocity.shape) != spatial + (D,)):
         return False
     o = nat.MacroscopicOut()
     o.dtype = nat.F64 if fields[0].dtype == torch.float64 else nat.F32
@@ -232,8 +192,11 @@ def _get_in_place(ctx, pdfs, density, velocity, code, density_deviation):
         if t is not None:
             setattr(o, name, t[inner].data_ptr())
     d = ctx.descriptor(pdfs)
-    nat.check(nat.load().lbm355_get_fields(ctypes.byref(d), ctypes.c_void_p(pdfs.data_ptr()), ctypes.byref(o), code,
-                                           nat.current_stream_handle()))
+    lib = nat.load()
+    if not lib.lbm355_fields_apart(ctypes.byref(d), pdfs.data_ptr(), ctypes.byref(o)):
+        return False
+    nat.check(lib.lbm355_get_fields(ctypes.byref(d), ctypes.c_void_p(pdfs.data_ptr()), ctypes.byref(o), code,
+                                    nat.current_stream_handle()))
     torch.autograd.graph.increment_version(fields)   # as torch's own writes do, for what autograd saved
     return True
 

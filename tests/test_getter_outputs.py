@@ -1,10 +1,41 @@
 """The macroscopic getter writes its outputs directly only where every element written is its own."""
+import ctypes
+import os
+
 import pytest
 import torch
 
-from lbmpy_amd.macroscopic_value_kernels import _own_memory
+from lbmpy_amd import _native as nat
 
 SHAPE = (6, 5, 4)
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _library():
+    from lbmpy_amd.csrc.build import library_path
+    if not os.path.exists(library_path()):
+        pytest.skip("liblbm355.so not built (run __graft_entry__.build())")
+
+
+def _own_memory(pdfs, scalars, velocity):
+    """lbm355_fields_apart for these tensors (host code, which reads no element)."""
+    D = pdfs.dim() - 1
+    d, o = nat.SweepDesc(), nat.MacroscopicOut()
+    d.stencil = nat.D2Q9 if D == 2 else nat.D3Q19
+    d.store_dtype = o.dtype = nat.F32
+    d.nx, d.ny, d.nz = tuple(pdfs.shape[:D]) + (1,) * (3 - D)
+    d.stride_y, d.stride_z, d.stride_q = pdfs.stride(1), pdfs.stride(2) if D == 3 else 0, pdfs.stride(D)
+    for name, t in zip(("density", "density_deviation"), scalars):
+        setattr(o, name, t.data_ptr())
+        assert t.stride() == scalars[0].stride()
+        for a in range(D):
+            o.scalar_stride[a] = t.stride(a)
+    if velocity is not None:
+        o.velocity = velocity.data_ptr()
+        for a in range(D):
+            o.vector_stride[a] = velocity.stride(a)
+        o.vector_stride[3] = velocity.stride(D)
+    return bool(nat.load().lbm355_fields_apart(ctypes.byref(d), pdfs.data_ptr(), ctypes.byref(o)))
 
 
 def _pdfs(q=19, extra=0):
@@ -33,6 +64,10 @@ def test_interleaved_components_are_separate():
     assert _own_memory(_pdfs(), [cell[..., 3]], cell[..., :3])
     plane = _f(*SHAPE, 5)                      # one x-fastest plane per component
     assert _own_memory(_pdfs(), [plane[..., 0], plane[..., 4]], plane[..., 1:4])
+    flat = torch.zeros(9, 7, 6).permute(2, 1, 0)
+    cell = _c(6, 7, 3)
+    assert _own_memory(flat, [cell[..., 0]], cell[..., 1:]) and _own_memory(flat, [_f(6, 7)], _c(6, 7, 2))
+    assert not _own_memory(flat, [cell[..., 1]], cell[..., 1:])
     padded = torch.zeros(SHAPE[0] + 2, SHAPE[1], SHAPE[2] + 3)
     assert _own_memory(_pdfs(), [padded[1:-1, :, :SHAPE[2]]], None)
 
