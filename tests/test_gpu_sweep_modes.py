@@ -203,3 +203,49 @@ def test_refusals():
     run = (lambda access: lib.lbm355_sweep_with_access(d, pdf.data_ptr(), pdf.data_ptr(), None, None, access, None))
     assert run(nat.ACCESS_ROWS) == run(nat.ACCESS_WAVES) == 2 and run(-1) == 1 and run(5) == 2
     assert float(pdf.abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("pattern,mode", [("pull", "rows"), ("push", "rows"), ("esopull", "rows"), ("pull", "waves")])
+def test_padded_rows_on_lines(pattern, mode):
+    """Rows with ghost layers and padding, whose cells start on lines, are streamed; without padding they are not."""
+    family, dtype = ("cumulant", "float32") if mode == "rows" else ("D3Q19-mrt", "float16")
+    nx, ny, nz, q = (128, 120, 100, 27) if mode == "rows" else (128, 160, 160, 19)
+    if pattern == "esopull":
+        nx, ny, nz = 256, 192, 160
+    ks = _kernels(family, pattern, dtype, 1)
+    for k in ks:
+        k.set_faces(["periodic"] * 3)
+    per_line = 128 // torch.empty(0, dtype=getattr(torch, dtype)).element_size()
+    full = (nx + 2, ny + 2, nz + 2)
+
+    def arrays(padded):
+        sy = -(-full[0] // per_line) * per_line if padded else full[0]
+        sz = sy * full[1]
+        sq = sz * full[2]
+        first = -(1 + sy + sz) % per_line if padded else 0
+        out = []
+        for _ in range(2 if pattern in ("pull", "push") else 1):
+            flat = torch.zeros(q * sq + first, dtype=getattr(torch, dtype), device="cuda")
+            out.append(flat.as_strided(full + (q,), (1, sy, sz, sq), first))
+        return out
+
+    g = torch.Generator(device="cuda").manual_seed(5)
+    state = 1e-2 * torch.randn((nx, ny, nz, q), generator=g, device="cuda")
+    results = []
+    for padded in (True, False):
+        a = arrays(padded)
+        a[0][1:-1, 1:-1, 1:-1] = state.to(a[0].dtype)
+        chosen = set()
+        for s in range(2):
+            k = ks[s % len(ks)]
+            chosen.add(nat.load().lbm355_sweep_access(k.descriptor(a[0], {}), a[0].data_ptr(), a[-1].data_ptr()))
+            if len(a) == 2:
+                k(src=a[0], dst=a[1])
+                a = a[::-1]
+            else:
+                k(src=a[0])
+        assert chosen == ({MODES[mode]} if padded else {nat.ACCESS_SHARED})
+        results.append(a[0][1:-1, 1:-1, 1:-1].double())
+    tol = 128 * EPS[dtype] * float(results[1].abs().max()) + (2.0 ** -10 * float(results[1].abs().max())
+                                                              if dtype == "float16" else 0.0)
+    assert float((results[0] - results[1]).abs().max()) <= tol and float((results[1] - state).abs().max()) > 1e-3
